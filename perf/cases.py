@@ -73,7 +73,7 @@ def listed():
         _case("air5-40x33x29", "chain", 40, 33, 29, gas="air5", steps=30, flow=True),
         _case("air5-96", "chain", 96, 96, 96, gas="air5", steps=60),
         _case("air5-128-mixed", "chain", 128, 128, 128, gas="air5", precision="mixed", steps=50),
-        _case("air5-chain-6-of-45", "chain", 45, 52, 40, nb=6, gas="air5", steps=50),
+        _case("air5-chain-4-of-45", "chain", 45, 52, 40, nb=4, gas="air5", steps=30),
     ]
 
 
@@ -110,8 +110,8 @@ def draw(rng):
         return _case(None, "chain", *n, gas="air5", flux=rng.choice(["ausmdv", "hllc"]), scheme=rng.choice(["pc", "euler"]),
                      precision=rng.choice(["fp64", "fp64", "mixed"]), steps=rng.randint(25, 45))
     n = box(120000)
-    return _case(None, "chain", *n, nb=rng.randint(3, 8), gas="air5", flux="ausmdv",
-                 precision=rng.choice(["fp64", "mixed"]), steps=rng.randint(25, 45))
+    return _case(None, "chain", *n, nb=rng.randint(2, 4), gas="air5", flux="ausmdv",
+                 precision=rng.choice(["fp64", "mixed"]), steps=rng.randint(20, 32))
 
 
 # ------------------------------------------------------------------- inputs
