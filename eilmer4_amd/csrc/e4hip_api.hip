@@ -908,7 +908,8 @@ int launch_stage_batch(const std::vector<const BlockH*>& blks, const std::vector
 // Whether a mixture can use the fast modes' mixture form (tp_gas_device.h).
 bool tp_mixture_form(const e4::TPGas& g)
 {
-    return g.shared != 0 && g.curve[0].nseg == e4::TP_FAST_NSEG;
+    return g.shared != 0 && g.curve[0].nseg == e4::TP_FAST_NSEG && g.Tlo <= g.blo[0] && g.bhi[0] < g.blo[1] &&
+           g.bhi[1] <= g.Thi;
 }
 
 // The thermally perfect kernels' arguments for one block's stage.
@@ -1353,6 +1354,17 @@ int e4hip_gas_tp(int nsp, const double* M, int nseg, const double* Tbreaks, cons
     for (int q = 0; q < nseg; ++q)
         for (int k = 0; k < 8; ++k)
             for (int s = 0; s < nsp; ++s) g.tp.RC[q][k][s] = g.tp.R[s] * g.tp.curve[s].c[q][k];
+    {
+        const e4::CeaCurve& c0 = g.tp.curve[0];
+        g.tp.Tlo = c0.Tb[0];
+        g.tp.Thi = c0.Tb[nseg];
+        for (int q = 0; q < 2; ++q) {
+            const bool blend = q < nseg - 1;
+            g.tp.blo[q] = blend ? c0.Tb[q + 1] - 0.5 * c0.Tbl[q] : g.tp.Thi;
+            g.tp.bhi[q] = blend ? c0.Tb[q + 1] + 0.5 * c0.Tbl[q] : g.tp.Thi;
+            g.tp.br[q] = (blend && c0.Tbl[q] > 0.0) ? 1.0 / c0.Tbl[q] : 1.0e300;
+        }
+    }
     HIP_TRY(hipMalloc(&g.tp_dev, sizeof(e4::TPGas)));
     HIP_TRY(hipMemcpy(g.tp_dev, &g.tp, sizeof(e4::TPGas), hipMemcpyHostToDevice));
     {

@@ -220,7 +220,7 @@ __device__ __forceinline__ void gen_flux(const TPArgs& A, const GSide<NSP>& L, c
         for (int q = 0; q < 3; ++q) { Lc.v[q] = L.v[q]; Rc.v[q] = Rt.v[q]; }
 #pragma unroll
         for (int q = 0; q < NSP; ++q) { Lc.Y[q] = L.Y[q]; Rc.Y[q] = Rt.Y[q]; }
-        tp_flux<MA, NSP, FLUX>(A, *A.gas, Lc, Rc, shock, F);
+        tp_flux<MA, NSP, FLUX>(A, tp_gas(A), Lc, Rc, shock, F);
     }
 }
 
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(128) void gen_face_kernel(TPArgs A)
                     Q.T = tp_val(rc, P_T);
 #pragma unroll
                     for (int s = 0; s < NSP; ++s) Q.Y[s] = sd ? Rf.Y[s] : Lf.Y[s];
-                    if (tp_face_eos<MA, NSP, kPolish>(*A.gas, Q, &fe, &fb) == 0) {
+                    if (tp_face_eos<MA, NSP, kPolish>(tp_gas(A), Q, &fe, &fb) == 0) {
                         const double a = tp_val(rc, P_A);
                         if (sd == 0) { Lf.T = Q.T; Lf.u = Q.u; Lf.p = Q.p; Lf.a = a; okL = true; }
                         else { Rf.T = Q.T; Rf.u = Q.u; Rf.p = Q.p; Rf.a = a; okR = true; }

@@ -118,9 +118,9 @@ __device__ __forceinline__ float mlp_guess_wave(const GuessModel& G, const doubl
 // Newton steps with the reference's dzdT, sum_s Y_s (Cp_s - R_s), which inside a blend is not the
 // derivative of the blended energy (convergence there is only linear, hence a
 // test on the residual rather than on the size of the last step).
-template <class M, int NSP, class MX>
-__device__ __forceinline__ int tp_polish_x(const TPGas& g, const MX& X, double Rmix, TPState<NSP>& Q, double e_tgt,
-                                           double T0, int* fevals)
+template <class M, int NSP>
+__device__ __forceinline__ int tp_polish_x(const TPGas& g, double Rmix, TPState<NSP>& Q, double e_tgt, double T0,
+                                           int* fevals)
 {
     using MD = typename std::conditional<M::kFast, ModeFast64, ModeExact>::type;
     if (!(T0 >= 20.0 && T0 <= 100000.0)) return -1;
@@ -130,7 +130,7 @@ __device__ __forceinline__ int tp_polish_x(const TPGas& g, const MX& X, double R
         for (int it = 0;; ++it) {
             if (it == 2 && !(T >= 20.0 && T <= 100000.0)) return -1;
             double u, du, d2u;
-            tp_mix_eval<true>(X, g.curve[0], Rmix, T, &u, &du, &d2u);
+            tp_mix_eval_y<true, NSP>(g, Q.Y, Rmix, T, &u, &du, &d2u);
             (*fevals)++;
             const double f = u - e_tgt;
             if (it == 2) {
@@ -142,7 +142,7 @@ __device__ __forceinline__ int tp_polish_x(const TPGas& g, const MX& X, double R
             const double s = dv<MD>(2.0 * f * du, 2.0 * du * du - f * d2u);
             const double Tn = T - s;
             if (fabs(s) <= 1.0e-4 * Tn && Tn >= 20.0 && Tn <= 100000.0 &&
-                tp_curve_piece(g.curve[0], Tn) == tp_curve_piece(g.curve[0], T)) {
+                tp_curve_piece(g, Tn) == tp_curve_piece(g, T)) {
                 Q.T = Tn;
                 Q.u = e_tgt;
                 return 0;
@@ -173,13 +173,7 @@ __device__ __forceinline__ int tp_polish_x(const TPGas& g, const MX& X, double R
 template <class M, int NSP>
 __device__ __forceinline__ int tp_polish(const TPGas& g, TPState<NSP>& Q, double e_tgt, double T0, int* fevals)
 {
-    if constexpr (M::kFast) {
-        const TPMixY<NSP> X = tp_mix_y<NSP>(g, Q.Y);
-        return tp_polish_x<M, NSP>(g, X, tp_Rmix<NSP>(g, Q.Y), Q, e_tgt, T0, fevals);
-    } else {
-        TPMix X;   // unused by the reference form
-        return tp_polish_x<M, NSP>(g, X, 0.0, Q, e_tgt, T0, fevals);
-    }
+    return tp_polish_x<M, NSP>(g, M::kFast ? tp_Rmix<NSP>(g, Q.Y) : 0.0, Q, e_tgt, T0, fevals);
 }
 
 } // namespace e4

@@ -65,7 +65,34 @@ struct TPGas {
     double R[TP_NSP_MAX];
     CeaCurve curve[TP_NSP_MAX];
     double RC[TP_NSEG_MAX][8][TP_NSP_MAX];        // R_s a_{s,k} of segment q: RC[q][k][s]
+    // the shared curve of the fast modes: its range, and of its two blend
+    // ranges the ends and the reciprocal width (1e300 for one of no width)
+    double Tlo, Thi;
+    double blo[2], bhi[2], br[2];
 };
+
+// The gas model through a pointer to constant memory that the optimiser cannot
+// trace: its tables are the same in every lane and no kernel writes them.  The
+// address space makes their reads scalar loads whatever the kernel stores
+// before them (otherwise a store that might alias turns them into vector
+// loads), and an opaque pointer per curve evaluation keeps them inside the
+// loop of a solve (hoisted out of it they overflow the scalar registers and
+// come back lane by lane through vector registers: 142 -> 200 us per face
+// kernel at 96^3).
+__device__ __forceinline__ const TPGas& tp_gas_const(const TPGas* g)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    using KGas = const __attribute__((address_space(4))) TPGas*;
+    const unsigned long long b = (unsigned long long)g;
+    const unsigned int lo = (unsigned int)__builtin_amdgcn_readfirstlane((int)(unsigned int)b);
+    const unsigned int hi = (unsigned int)__builtin_amdgcn_readfirstlane((int)(unsigned int)(b >> 32));
+    KGas p = (KGas)(((unsigned long long)hi << 32) | lo);
+    asm volatile("" : "+s"(p));
+    return *(const TPGas*)p;
+#else
+    return *g;
+#endif
+}
 
 template <int NSP>
 struct TPState {
@@ -228,56 +255,19 @@ __device__ __forceinline__ void tp_mix_u_cv(const TPGas& g, const double* Y, dou
 // the same breakpoints; other mixtures run the reference-form kernels.
 constexpr int TP_FAST_NSEG = 3;
 
-// The mixture's coefficient sums of every segment, M[q][k] = sum_s Y_s R_s
-// a_{s,q,k}: formed once per temperature solve (the composition is fixed
-// during the solve), so an evaluation at any T only weights the three sets.
-struct TPMix {
-    double M[TP_FAST_NSEG][8];
+// Weights of the three segments at Tc: one segment, or the linear blend of
+// two inside a blend range (cea_thermo_curves.d:136-169).  b1 and b2 are how
+// far Tc is through each blend range, clamped to [0, 1] by the multiply's own
+// output modifier; the weights are their differences, without a comparison or
+// a select (they were some 40 instructions of every curve evaluation).
+struct TPWeights {
+    double b1, b2;
+    __device__ __forceinline__ double w(int q) const { return q == 0 ? 1.0 - b1 : (q == 1 ? b1 - b2 : b2); }
 };
-
-template <int NSP>
-__device__ __forceinline__ void tp_mix_all(const TPGas& g, const double* Y, TPMix& X)
+__device__ __forceinline__ double unit_clamp(double x) { return fmin(fmax(x, 0.0), 1.0); }
+__device__ __forceinline__ TPWeights tp_seg_weights(const TPGas& g, double Tc)
 {
-#pragma unroll
-    for (int q = 0; q < TP_FAST_NSEG; ++q)
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            double m = 0.0;
-#pragma unroll
-            for (int s = 0; s < NSP; ++s) m += Y[s] * g.RC[q][k][s];
-            X.M[q][k] = m;
-        }
-}
-
-// A value that is the same in every lane of the wave (here: a field of the
-// gas model, whose address is uniform), pinned to a scalar register: without
-// this the compiler may turn a per-lane choice between two such fields into
-// a per-lane load, a memory round trip inside every curve evaluation.
-__device__ __forceinline__ double uniform_f64(double x)
-{
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
-    const unsigned int lo = (unsigned int)__builtin_amdgcn_readfirstlane((int)(unsigned int)b);
-    const unsigned int hi = (unsigned int)__builtin_amdgcn_readfirstlane((int)(unsigned int)(b >> 32));
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
-// Weights of the three segments at Tc and their T derivatives: one segment,
-// or the linear blend of two inside a blend range (cea_thermo_curves.d:136-169,
-// the same comparisons).
-__device__ __forceinline__ void tp_seg_weights(const CeaCurve& cv, double Tc, double w[3], double dw[3])
-{
-    const double lo1 = uniform_f64(cv.Tb[1] - 0.5 * cv.Tbl[0]), hi1 = uniform_f64(cv.Tb[1] + 0.5 * cv.Tbl[0]);
-    const double lo2 = uniform_f64(cv.Tb[2] - 0.5 * cv.Tbl[1]), hi2 = uniform_f64(cv.Tb[2] + 0.5 * cv.Tbl[1]);
-    const double r1 = uniform_f64(cv.rTbl[0]), r2 = uniform_f64(cv.rTbl[1]);
-    const bool in1 = Tc >= lo1 && Tc <= hi1, in2 = Tc >= lo2 && Tc <= hi2;
-    const double wb = in1 ? r1 * (Tc - lo1) : r2 * (Tc - lo2);
-    const double rb = in1 ? r1 : r2;
-    w[0] = (Tc < lo1) ? 1.0 : (in1 ? 1.0 - wb : 0.0);
-    w[1] = in1 ? wb : (in2 ? 1.0 - wb : ((Tc > hi1 && Tc < lo2) ? 1.0 : 0.0));
-    w[2] = in2 ? wb : ((Tc > hi2) ? 1.0 : 0.0);
-    dw[0] = in1 ? -rb : 0.0;
-    dw[1] = in1 ? rb : (in2 ? -rb : 0.0);
-    dw[2] = in2 ? rb : 0.0;
+    return TPWeights{unit_clamp((Tc - g.blo[0]) * g.br[0]), unit_clamp((Tc - g.blo[1]) * g.br[1])};
 }
 
 // Which smooth piece of the fast modes' curve T lies on: below the curve
@@ -286,87 +276,51 @@ __device__ __forceinline__ void tp_seg_weights(const CeaCurve& cv, double Tc, do
 // comparisons as tp_seg_weights.  On one piece the energy is one smooth
 // expression of T (a segment's polynomial and log terms, their linear blend,
 // or the constant-Cp extension).
-__device__ __forceinline__ int tp_curve_piece(const CeaCurve& cv, double T)
+__device__ __forceinline__ int tp_curve_piece(const TPGas& g, double T)
 {
-    if (T < uniform_f64(cv.Tb[0])) return 0;
-    if (T > uniform_f64(cv.Tb[TP_FAST_NSEG])) return 6;
-    const double lo1 = uniform_f64(cv.Tb[1] - 0.5 * cv.Tbl[0]), hi1 = uniform_f64(cv.Tb[1] + 0.5 * cv.Tbl[0]);
-    const double lo2 = uniform_f64(cv.Tb[2] - 0.5 * cv.Tbl[1]), hi2 = uniform_f64(cv.Tb[2] + 0.5 * cv.Tbl[1]);
-    if (T < lo1) return 1;
-    if (T <= hi1) return 2;
-    if (T < lo2) return 3;
-    if (T <= hi2) return 4;
-    return 5;
+    return (T >= g.Tlo) + (T >= g.blo[0]) + (T > g.bhi[0]) + (T >= g.blo[1]) + (T > g.bhi[1]) + (T > g.Thi);
 }
 
-// u, du/dT and d2u/dT2 of the mixture at T from its segment sums.  SLOPE:
+// u, du/dT and d2u/dT2 of the mixture at T (fast modes).  SLOPE:
 // du/dT is the exact derivative of the blended curve, which inside a blend
 // adds (dw_B/dT)(h_B - h_A) to the blended Cv; without it du/dT is the blended
 // Cv (the reference's dzdT, therm_perf_gas_mix_eos.d:116-123) and d2u is not
 // formed.  Outside the curve range: the constant-Cp extension
 // (cea_thermo_curves.d:63-91).
-template <bool SLOPE>
-__device__ __forceinline__ void tp_mix_eval(const TPMix& X, const CeaCurve& c0, double Rmix, double T, double* u,
-                                            double* du, double* d2u)
-{
-    const double Tlo = uniform_f64(c0.Tb[0]), Thi = uniform_f64(c0.Tb[TP_FAST_NSEG]);
-    const double Tc = fmin(fmax(T, Tlo), Thi);
-    double w[3], dw[3];
-    tp_seg_weights(c0, Tc, w, dw);
-    double Mk[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) Mk[k] = w[0] * X.M[0][k] + w[1] * X.M[1][k] + w[2] * X.M[2][k];
-    const double r = dv_seed(1.0, Tc, rcp_seed(Tc));
-    const double lnT = log_fast(Tc);
-    const double T2 = Tc * Tc, T3 = T2 * Tc, T4 = T2 * T2;
-    double h = tp_mix_h(Mk, Tc, r, lnT);
-    const double cp = Mk[0] * r * r + Mk[1] * r + Mk[2] + Mk[3] * Tc + Mk[4] * T2 + Mk[5] * T3 + Mk[6] * T4;
-    double dh = cp, d2h = 0.0;
-    if constexpr (SLOPE) {
-        d2h = -2.0 * Mk[0] * r * r * r - Mk[1] * r * r + Mk[3] + 2.0 * Mk[4] * Tc + 3.0 * Mk[5] * T2 +
-              4.0 * Mk[6] * T3;
-        if (dw[0] != 0.0 || dw[1] != 0.0 || dw[2] != 0.0) {
-            double dM[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) dM[k] = dw[0] * X.M[0][k] + dw[1] * X.M[1][k] + dw[2] * X.M[2][k];
-            dh += tp_mix_h(dM, Tc, r, lnT);
-            d2h += 2.0 * (dM[0] * r * r + dM[1] * r + dM[2] + dM[3] * Tc + dM[4] * T2 + dM[5] * T3 + dM[6] * T4);
-        }
-    }
-    if (T < Tlo) { h -= cp * (Tlo - T); dh = cp; d2h = 0.0; }
-    else if (T > Thi) { h += cp * (T - Thi); dh = cp; d2h = 0.0; }
-    *u = h - Rmix * T;
-    *du = dh - Rmix;
-    *d2u = d2h;
-}
-
-// tp_mix_eval from the mass fractions instead of tp_mix_all's sums: each
-// evaluation forms the species sums of the segments that some lane of the
-// wave weights (a wave-uniform test), so that a solve keeps NSP mass
-// fractions in registers instead of all the segments' sums.  Per lane the
-// arithmetic is that of tp_mix_eval: a segment no lane weights would add
-// w * M = 0.
+//
+// Each evaluation forms the species sums of the segments that some lane of the
+// wave weights (a wave-uniform test), so that a solve keeps NSP mass fractions
+// in registers instead of all the segments' sums.
 template <bool SLOPE, int NSP>
-__device__ __forceinline__ void tp_mix_eval_y(const TPGas& g, const double* Y, double Rmix, double T, double* u,
+__device__ __forceinline__ void tp_mix_eval_y(const TPGas& gas, const double* Y, double Rmix, double T, double* u,
                                               double* du, double* d2u)
 {
-    const CeaCurve& c0 = g.curve[0];
-    const double Tlo = uniform_f64(c0.Tb[0]), Thi = uniform_f64(c0.Tb[TP_FAST_NSEG]);
-    const double Tc = fmin(fmax(T, Tlo), Thi);
-    double w[3], dw[3];
-    tp_seg_weights(c0, Tc, w, dw);
+    const TPGas& g = tp_gas_const(&gas);
+    const double Tc = fmin(fmax(T, g.Tlo), g.Thi);
+    const TPWeights W = tp_seg_weights(g, Tc);
+    double dw[3] = {0.0, 0.0, 0.0};
+    bool in1 = false, in2 = false;
+    if constexpr (SLOPE) {
+        in1 = W.b1 > 0.0 && W.b1 < 1.0;
+        in2 = W.b2 > 0.0 && W.b2 < 1.0;
+        const double d1 = in1 ? g.br[0] : 0.0, d2 = in2 ? g.br[1] : 0.0;
+        dw[0] = -d1;
+        dw[1] = d1 - d2;
+        dw[2] = d2;
+    }
     double Mk[8], dM[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) { Mk[k] = 0.0; dM[k] = 0.0; }
 #pragma unroll
     for (int q = 0; q < TP_FAST_NSEG; ++q) {
-        if (__ballot(w[q] != 0.0 || (SLOPE && dw[q] != 0.0)) == 0) continue;
+        const double w = W.w(q);
+        if (__ballot(w != 0.0) == 0) continue;   // a lane inside a blend weights both its segments
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             double m = 0.0;
 #pragma unroll
             for (int s = 0; s < NSP; ++s) m += Y[s] * g.RC[q][k][s];
-            Mk[k] += w[q] * m;
+            Mk[k] += w * m;
             if constexpr (SLOPE) dM[k] += dw[q] * m;
         }
     }
@@ -379,43 +333,19 @@ __device__ __forceinline__ void tp_mix_eval_y(const TPGas& g, const double* Y, d
     if constexpr (SLOPE) {
         d2h = -2.0 * Mk[0] * r * r * r - Mk[1] * r * r + Mk[3] + 2.0 * Mk[4] * Tc + 3.0 * Mk[5] * T2 +
               4.0 * Mk[6] * T3;
-        if (dw[0] != 0.0 || dw[1] != 0.0 || dw[2] != 0.0) {
+        if (in1 || in2) {
             dh += tp_mix_h(dM, Tc, r, lnT);
             d2h += 2.0 * (dM[0] * r * r + dM[1] * r + dM[2] + dM[3] * Tc + dM[4] * T2 + dM[5] * T3 + dM[6] * T4);
         }
     }
-    if (T < Tlo) { h -= cp * (Tlo - T); dh = cp; d2h = 0.0; }
-    else if (T > Thi) { h += cp * (T - Thi); dh = cp; d2h = 0.0; }
+    // the constant-Cp extension; a wave inside the range skips it
+    if (__ballot(T != Tc) != 0) {
+        h += cp * (T - Tc);
+        if (T != Tc) { dh = cp; d2h = 0.0; }
+    }
     *u = h - Rmix * T;
     *du = dh - Rmix;
     *d2u = d2h;
-}
-
-// The composition as the fast solves see it through tp_mix_eval: TPMix, the
-// segment sums formed once per solve, or TPMixY, the mass fractions with the
-// sums formed at each evaluation (tp_mix_eval_y: fewer registers held through
-// the solve, more arithmetic per evaluation).
-template <int NSP>
-struct TPMixY {
-    const TPGas* g;
-    double Y[NSP];
-};
-
-template <int NSP>
-__device__ __forceinline__ TPMixY<NSP> tp_mix_y(const TPGas& g, const double* Y)
-{
-    TPMixY<NSP> X;
-    X.g = &g;
-#pragma unroll
-    for (int s = 0; s < NSP; ++s) X.Y[s] = Y[s];
-    return X;
-}
-
-template <bool SLOPE, int NSP>
-__device__ __forceinline__ void tp_mix_eval(const TPMixY<NSP>& X, const CeaCurve&, double Rmix, double T, double* u,
-                                            double* du, double* d2u)
-{
-    tp_mix_eval_y<SLOPE, NSP>(*X.g, X.Y, Rmix, T, u, du, d2u);
 }
 
 // therm_perf_gas_mix_eos.d:63-69 (mass_average, gas_model.d:330-338)
@@ -478,11 +408,10 @@ __device__ __forceinline__ void tp_u_dzdT(const TPGas& g, const double* Y, doubl
 // All energy evaluations (the two bracket ends, then the iterates from x0)
 // go through one call site in one loop, which keeps the inlined code to one
 // copy of the energy evaluation.
-template <class M, int NSP, class MX>
-__device__ __forceinline__ int tp_newton(const TPGas& g, const MX& X, double Rmix, TPState<NSP>& Q, double e_tgt,
-                                         double x0, double xMin, double xMax, double tol, double* root, int* fevals)
+template <class M, int NSP>
+__device__ __forceinline__ int tp_newton(const TPGas& g, TPState<NSP>& Q, double e_tgt, double x0, double xMin,
+                                         double xMax, double tol, double* root, int* fevals)
 {
-    using MD = typename std::conditional<M::kFast, ModeFast64, ModeExact>::type;
     const int MAXIT = 30;
     double xL = xMin, xH = xMax, fL = 0.0;
     double rts = x0;
@@ -493,13 +422,7 @@ __device__ __forceinline__ int tp_newton(const TPGas& g, const MX& X, double Rmi
         // evaluation n: 0 the lower bracket end, 1 the upper, 2+ the iterates
         const double T = (n == 0) ? xMin : (n == 1) ? xMax : rts;
         double u, df0;
-        if constexpr (M::kFast) {
-            double du, d2u;
-            tp_mix_eval<false>(X, g.curve[0], Rmix, T, &u, &du, &d2u);
-            df0 = -1.0 * du;
-        } else {
-            tp_u_dzdT<M, NSP>(g, Q.Y, T, n >= 2, &u, &df0);
-        }
+        tp_u_dzdT<M, NSP>(g, Q.Y, T, n >= 2, &u, &df0);
         Q.T = T;
         Q.u = u;
         (*fevals)++;
@@ -523,7 +446,7 @@ __device__ __forceinline__ int tp_newton(const TPGas& g, const MX& X, double Rmi
             if (xL == rts) { *root = rts; return 0; }
         } else {
             dxold = dx;
-            dx = dv<MD>(f0, df0);
+            dx = dv<M>(f0, df0);
             double tmp = rts;
             rts -= dx;
             if (tmp == rts) { *root = rts; return 0; }
@@ -532,30 +455,129 @@ __device__ __forceinline__ int tp_newton(const TPGas& g, const MX& X, double Rmi
     }
 }
 
+// tp_newton's iterate sequence in the fast modes.  The energies of the bracket
+// ends, which tp_newton evaluates first, only decide whether the bracket holds
+// a root and which end is the low one.  With u(T) increasing, iterates that
+// never bisect and end more than 1e-3 K inside the bracket have shown both, so
+// the ends are evaluated only when some lane of the wave wants its first
+// bisection, or has ended near an end: 3.1 evaluations a solve instead of 5.1
+// on five-species air at 300-8000 K (with the cheaper segment weights, face
+// kernels at 96^3 in FP64 142 -> 112 us, the update 130 -> 120 us; issue-bound).
+// Every lane of the wave goes through the same straight-line body, a finished lane keeping its values: lane-wise exits
+// cost more register copies than the evaluations they saved.  f = e_tgt - u is
+// taken to fall from xMin to xMax, or with `rising` to rise.  Returns 0 with Q.T
+// the root and Q.u the energy of the last iterate, -1 where tp_newton would
+// throw, and 1 where the ends show the order to be the other one.
+template <int NSP>
+__device__ __forceinline__ int tp_newton_fast(const TPGas& g, TPState<NSP>& Q, double Rmix, double e_tgt, double x0,
+                                              double xMin, double xMax, bool rising, double tol, int* fevals)
+{
+    const int MAXIT = 30;
+    double T = x0, ulast = 0.0, fL = 0.0;
+    double xL = rising ? xMin : xMax, xH = rising ? xMax : xMin;
+    double dxold = xMax - xMin, dx = dxold;
+    bool live = true;                        // still iterating
+    bool known = rising;                     // the ends are known to bracket a root
+    int rc = 0, j = 0;                       // j: Newton steps taken
+    int end = 0;                             // wave-uniform: 0 iterates, 1 the lower end, 2 the upper
+#pragma nounroll
+    for (;;) {
+        double u, du, d2u;
+        tp_mix_eval_y<false, NSP>(g, Q.Y, Rmix, (end == 0) ? T : (end == 1) ? xMin : xMax, &u, &du, &d2u);
+        const double f0 = e_tgt - u;
+        if (end == 0) {
+            bool ask = false;                // a bisection has to wait for the ends
+            if (live) {
+                (*fevals)++;
+                ulast = u;
+                const double df0 = -1.0 * du;
+                if (j > 0) {
+                    xL = (f0 < 0.0) ? T : xL;
+                    xH = (f0 < 0.0) ? xH : T;
+                }
+                const bool bisect = (((T - xH) * df0 - f0) * ((T - xL) * df0 - f0) > 0.0) ||
+                                    (fabs(2.0 * f0) > fabs(dxold * df0));
+                ask = bisect && !known;
+                if (j == MAXIT) {
+                    live = false;
+                    rc = -1;
+                } else if (!ask) {
+                    dxold = dx;
+                    dx = dv<ModeFast64>(f0, df0);
+                    double from = T, to = T - dx;
+                    if (__builtin_expect(bisect, 0)) {
+                        dx = 0.5 * (xH - xL);
+                        from = xL;
+                        to = xL + dx;
+                    }
+                    T = to;
+                    live = !(from == to || fabs(dx) < tol);
+                    // a root beside an end has to wait for the ends, too
+                    ask = !live && !known && !(T > xMin + 1.0e-3 && T < xMax - 1.0e-3);
+                    ++j;
+                }
+            }
+            if (__ballot(ask) != 0) end = 1;
+            else if (__ballot(live) == 0) break;
+        } else if (end == 1) {
+            fL = f0;
+            end = 2;
+        } else {
+            if (rc == 0 && !known) {
+                (*fevals) += 2;
+                if ((fL > 0.0 && f0 > 0.0) || (fL < 0.0 && f0 < 0.0)) {
+                    rc = -1;
+                    live = false;
+                } else if (fL == 0.0 || f0 == 0.0) {
+                    T = (fL == 0.0) ? xMin : xMax;
+                    ulast = u;
+                    live = false;
+                } else if (fL < 0.0) {
+                    rc = 1;
+                    live = false;
+                }
+                known = true;
+            }
+            end = 0;
+            if (__ballot(live) == 0) break;
+        }
+    }
+    if (rc != 0) return rc;
+    Q.T = T;
+    Q.u = ulast;
+    return 0;
+}
+
 // therm_perf_gas_mix_eos.d:70-153: guess = Q.T, bracket [max(T-500, 20), +1000],
-// then [20, 1e5]; tolerance 1e-6 K.  X and Rmix: the composition's segment
-// sums and gas constant (fast modes; unused by ModeExact).
-template <class M, int NSP, class MX>
-__device__ __forceinline__ int tp_update_temperature_x(const TPGas& g, const MX& X, double Rmix, TPState<NSP>& Q,
-                                                       int* fevals)
+// then [20, 1e5]; tolerance 1e-6 K.  Rmix: the composition's gas constant (fast
+// modes; unused by ModeExact).
+template <class M, int NSP>
+__device__ __forceinline__ int tp_update_temperature_x(const TPGas& g, double Rmix, TPState<NSP>& Q, int* fevals)
 {
     const double Tsave = Q.T;
     const double e_tgt = Q.u;
     const double delT = 1000.0;
     const double T1 = fmax(Q.T - 0.5 * delT, 20.0);
+    bool rising = false;
 #pragma nounroll
-    for (int attempt = 0; attempt < 2; ++attempt) {
+    for (int attempt = 0; attempt < 2;) {
         const double lo = attempt ? 20.0 : T1, hi = attempt ? 100000.0 : T1 + delT;
-        double root;
-        if (tp_newton<M, NSP>(g, X, Rmix, Q, e_tgt, Tsave, lo, hi, 1.0e-6, &root, fevals) == 0) {
-            Q.T = root;
-            return 0;
+        int rc;
+        if constexpr (M::kFast) {
+            rc = tp_newton_fast<NSP>(g, Q, Rmix, e_tgt, Tsave, lo, hi, rising, 1.0e-6, fevals);
+        } else {
+            double root;
+            rc = tp_newton<M, NSP>(g, Q, e_tgt, Tsave, lo, hi, 1.0e-6, &root, fevals);
+            if (rc == 0) Q.T = root;
         }
+        if (rc == 0) return 0;
+        rising = rc > 0;
+        if (rc < 0) ++attempt;
     }
     Q.T = Tsave;
     if constexpr (M::kFast) {
         double du, d2u;
-        tp_mix_eval<false>(X, g.curve[0], Rmix, Tsave, &Q.u, &du, &d2u);
+        tp_mix_eval_y<false, NSP>(g, Q.Y, Rmix, Tsave, &Q.u, &du, &d2u);
     } else {
         Q.u = tp_energy<M, NSP>(g, Q.Y, Tsave);
     }
@@ -565,25 +587,17 @@ __device__ __forceinline__ int tp_update_temperature_x(const TPGas& g, const MX&
 template <class M, int NSP>
 __device__ __forceinline__ int tp_update_temperature(const TPGas& g, TPState<NSP>& Q, int* fevals)
 {
-    if constexpr (M::kFast) {
-        // the composition with its segment sums formed at each evaluation
-        // (fewer registers than holding all segments' sums through the solve)
-        const TPMixY<NSP> X = tp_mix_y<NSP>(g, Q.Y);
-        return tp_update_temperature_x<M, NSP>(g, X, tp_Rmix<NSP>(g, Q.Y), Q, fevals);
-    } else {
-        TPMix X;   // unused by the reference form
-        return tp_update_temperature_x<M, NSP>(g, X, 0.0, Q, fevals);
-    }
+    return tp_update_temperature_x<M, NSP>(g, M::kFast ? tp_Rmix<NSP>(g, Q.Y) : 0.0, Q, fevals);
 }
 
 // Frozen sound speed a = sqrt(Cp/Cv R T) (therm_perf_gas.d:345-385) from the
-// composition's segment sums (fast modes).
-template <class M, class MX>
-__device__ __forceinline__ double tp_sound_speed_x(const TPGas& g, const MX& X, double Rmix, double T)
+// mixture's curve (fast modes).
+template <class M, int NSP>
+__device__ __forceinline__ double tp_sound_speed_x(const TPGas& g, const double* Y, double Rmix, double T)
 {
     using MD = typename std::conditional<M::kFast, ModeFast64, ModeExact>::type;
     double u, cv, d2u;
-    tp_mix_eval<false>(X, g.curve[0], Rmix, T, &u, &cv, &d2u);
+    tp_mix_eval_y<false, NSP>(g, Y, Rmix, T, &u, &cv, &d2u);
     return sqrt(dv<MD>(cv + Rmix, cv) * (Rmix * T));
 }
 

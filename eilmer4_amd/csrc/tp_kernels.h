@@ -40,23 +40,22 @@ template <> struct TPFlux<ModeMixed> { using type = ModeMixed; };
 template <class M>
 using TPFluxStore = typename std::conditional<std::is_same<M, ModeMixed>::value, float, double>::type;
 
+// the block's gas model
+__device__ __forceinline__ const TPGas& tp_gas(const TPArgs& A) { return tp_gas_const(A.gas); }
+
 // update_thermo_from_rhou of a face state (therm_perf_gas.d:187-191); with
 // polish, Newton from Q.T first (*fallbacks counts the solves it hands on).
 template <class M, int NSP, bool POLISH>
 __device__ __forceinline__ int tp_face_eos(const TPGas& g, TPState<NSP>& Q, int* fevals, int* fallbacks)
 {
     if constexpr (M::kFast) {
-        // the composition for the polish and the bracketed solve, its
-        // segment sums formed at each evaluation: fewer registers in the face
-        // kernels (three waves per SIMD)
-        const TPMixY<NSP> X = tp_mix_y<NSP>(g, Q.Y);
         const double Rmix = tp_Rmix<NSP>(g, Q.Y);
         int rc = -1;
         if constexpr (POLISH) {
-            rc = tp_polish_x<M, NSP>(g, X, Rmix, Q, Q.u, Q.T, fevals);
+            rc = tp_polish_x<M, NSP>(g, Rmix, Q, Q.u, Q.T, fevals);
             if (rc != 0) (*fallbacks)++;
         }
-        if (rc != 0) rc = tp_update_temperature_x<M, NSP>(g, X, Rmix, Q, fevals);
+        if (rc != 0) rc = tp_update_temperature_x<M, NSP>(g, Rmix, Q, fevals);
         if (rc == 0) Q.p = Q.rho * Rmix * Q.T;
         return rc;
     } else {
@@ -88,7 +87,6 @@ __device__ __forceinline__ void tp_face_halley_pair(const TPGas& g, const double
                                                     double RR, double eL, double eR, double& TL, double& TR,
                                                     bool& okL, bool& okR, int* fevals)
 {
-    const CeaCurve& c0 = g.curve[0];
     bool liveL = TL >= 20.0 && TL <= 100000.0, liveR = TR >= 20.0 && TR <= 100000.0;
     okL = false;
     okR = false;
@@ -99,7 +97,7 @@ __device__ __forceinline__ void tp_face_halley_pair(const TPGas& g, const double
         const double f = u - e;
         const double s = dv<ModeFast64>(2.0 * f * du, 2.0 * du * du - f * d2u);
         const double tn = t - s;
-        if (tp_curve_piece(c0, tn) == tp_curve_piece(c0, t) && fabs(s) <= 1.0e-3 * tn && tn >= 20.0 &&
+        if (tp_curve_piece(g, tn) == tp_curve_piece(g, t) && fabs(s) <= 1.0e-3 * tn && tn >= 20.0 &&
             tn <= 100000.0) {
             out = tn;
             ok = true;
@@ -664,9 +662,9 @@ __device__ __forceinline__ void tp_face_body(const TPArgs& A, long f0)
             double YL[NSP], YR[NSP];
 #pragma unroll
             for (int s = 0; s < NSP; ++s) { YL[s] = double(Lf.Y[s]); YR[s] = double(Rf.Y[s]); }
-            const double RmL = tp_Rmix<NSP>(*A.gas, YL), RmR = tp_Rmix<NSP>(*A.gas, YR);
+            const double RmL = tp_Rmix<NSP>(tp_gas(A), YL), RmR = tp_Rmix<NSP>(tp_gas(A), YR);
             double TfL = TL, TfR = TR;
-            tp_face_halley_pair<NSP>(*A.gas, YL, YR, RmL, RmR, double(Lf.u), double(Rf.u), TfL, TfR, okL, okR, &fe);
+            tp_face_halley_pair<NSP>(tp_gas(A), YL, YR, RmL, RmR, double(Lf.u), double(Rf.u), TfL, TfR, okL, okR, &fe);
             if (okL) { Lf.T = R(TfL); Lf.p = R(double(Lf.rho) * RmL * TfL); Lf.a = R(aL); }
             if (okR) { Rf.T = R(TfR); Rf.p = R(double(Rf.rho) * RmR * TfR); Rf.a = R(aR); }
             defer = !(okL && okR);
@@ -681,7 +679,7 @@ __device__ __forceinline__ void tp_face_body(const TPArgs& A, long f0)
             Q.T = sd ? TR : TL;
 #pragma unroll
             for (int s = 0; s < NSP; ++s) Q.Y[s] = double(sd ? Rf.Y[s] : Lf.Y[s]);
-            if (tp_face_eos<MA, NSP, kPolish>(*A.gas, Q, &fe, &fb) == 0) {
+            if (tp_face_eos<MA, NSP, kPolish>(tp_gas(A), Q, &fe, &fb) == 0) {
                 const R a = R(sd ? aR : aL);
                 if (sd == 0) { Lf.T = R(Q.T); Lf.u = R(Q.u); Lf.p = R(Q.p); Lf.a = a; okL = true; }
                 else { Rf.T = R(Q.T); Rf.u = R(Q.u); Rf.p = R(Q.p); Rf.a = a; okR = true; }
@@ -708,7 +706,7 @@ __device__ __forceinline__ void tp_face_body(const TPArgs& A, long f0)
         if (!okR) Rf = tp_cell<NSP, R>(r[2], pn, pt1, pt2);
         R Fr[5 + NSP];
         const bool shock = (FLUX == FLUX_SHOCK) && ((r[1].s && *r[1].s) || (r[2].s && *r[2].s));
-        tp_flux<MF, NSP, FLUX>(A, *A.gas, Lf, Rf, shock, Fr);
+        tp_flux<MF, NSP, FLUX>(A, tp_gas(A), Lf, Rf, shock, Fr);
         using FS = TPFluxStore<M>;
         FS F[5 + NSP];
     #pragma unroll
@@ -922,41 +920,37 @@ __device__ __forceinline__ void tp_update_body(const TPArgs& A, long c)
         const double Tprev = A.Pin[P_T * qs + c];   // the previous temperature: the bracketed solve's guess
         int rc = -1;
         if constexpr (MA::kFast) {
-            // the composition for the polish, the bracketed solve and the sound
-            // speed, its segment sums formed at each evaluation from scalar
-            // loads of the gas tables: 111-115 VGPRs, four waves per SIMD
-            const TPMixY<NSP> X = tp_mix_y<NSP>(*A.gas, Q.Y);
-            const double Rmix = tp_Rmix<NSP>(*A.gas, Q.Y);
+            const double Rmix = tp_Rmix<NSP>(tp_gas(A), Q.Y);
             if constexpr (GUESS || kPolish) {
-                rc = tp_polish_x<MA, NSP>(*A.gas, X, Rmix, Q, e_tgt, GUESS ? Tguess : Tprev, &fe);
+                rc = tp_polish_x<MA, NSP>(tp_gas(A), Rmix, Q, e_tgt, GUESS ? Tguess : Tprev, &fe);
                 fell_back = rc != 0;
             }
             if (rc != 0) {
                 Q.u = e_tgt;
                 Q.T = Tprev;
-                rc = tp_update_temperature_x<MA, NSP>(*A.gas, X, Rmix, Q, &fe);
+                rc = tp_update_temperature_x<MA, NSP>(tp_gas(A), Rmix, Q, &fe);
             }
             if (rc == 0) {
                 Q.p = Q.rho * Rmix * Q.T;
-                Q.a = tp_sound_speed_x<MA>(*A.gas, X, Rmix, Q.T);
+                Q.a = tp_sound_speed_x<MA, NSP>(tp_gas(A), Q.Y, Rmix, Q.T);
             }
         } else {
             if constexpr (GUESS) {
-                rc = tp_polish<MA, NSP>(*A.gas, Q, e_tgt, Tguess, &fe);
-                if (rc == 0) Q.p = Q.rho * tp_Rmix<NSP>(*A.gas, Q.Y) * Q.T;
+                rc = tp_polish<MA, NSP>(tp_gas(A), Q, e_tgt, Tguess, &fe);
+                if (rc == 0) Q.p = Q.rho * tp_Rmix<NSP>(tp_gas(A), Q.Y) * Q.T;
                 else fell_back = true;
             }
             if (rc != 0) {
                 Q.u = e_tgt;
                 Q.T = Tprev;
-                rc = tp_update_thermo_from_rhou<MA, NSP>(*A.gas, Q, &fe);
+                rc = tp_update_thermo_from_rhou<MA, NSP>(tp_gas(A), Q, &fe);
             }
-            if (rc == 0) Q.a = tp_sound_speed<MA, NSP>(*A.gas, Q);
+            if (rc == 0) Q.a = tp_sound_speed<MA, NSP>(tp_gas(A), Q);
         }
         if (rc != 0) {
             // ignore_low_T_thermo_update_failure: T = 200 K and re-encode U
             Q.T = 200.0;
-            tp_update_thermo_from_rhoT<MA, NSP>(*A.gas, Q);
+            tp_update_thermo_from_rhoT<MA, NSP>(tp_gas(A), Q);
             // (integer stores, as above)
             unsigned long long* Un_out = reinterpret_cast<unsigned long long*>(A.Unew) + c;
             auto bits = [](double x) { return __builtin_bit_cast(unsigned long long, x); };
@@ -965,7 +959,7 @@ __device__ __forceinline__ void tp_update_body(const TPArgs& A, long c)
             Un_out[4 * qs] = bits(rho * (Q.u + ke2));
 #pragma unroll
             for (int s = 0; s < NSP; ++s) Un_out[(5 + s) * qs] = bits(rho * Q.Y[s]);
-            Q.a = tp_sound_speed<MA, NSP>(*A.gas, Q);
+            Q.a = tp_sound_speed<MA, NSP>(tp_gas(A), Q);
         }
         // check_data (flowstate.d:345-388)
         double fsum = 0.0;
@@ -1058,19 +1052,19 @@ __global__ __launch_bounds__(128) void tp_decode_kernel(TPArgs A, const double* 
         const double e_tgt = Q.u;
         int rc = -1;
         if (A.guess) {
-            rc = tp_polish<M, NSP>(*A.gas, Q, e_tgt, Tg, &fe);
-            if (rc == 0) Q.p = Q.rho * tp_Rmix<NSP>(*A.gas, Q.Y) * Q.T;
+            rc = tp_polish<M, NSP>(tp_gas(A), Q, e_tgt, Tg, &fe);
+            if (rc == 0) Q.p = Q.rho * tp_Rmix<NSP>(tp_gas(A), Q.Y) * Q.T;
             else fell_back = true;
         }
         if (rc != 0) {
             Q.u = e_tgt;
             Q.T = Tguess[c];
-            rc = tp_update_thermo_from_rhou<M, NSP>(*A.gas, Q, &fe);
+            rc = tp_update_thermo_from_rhou<M, NSP>(tp_gas(A), Q, &fe);
         }
         if (rc != 0) {
             bad = true;
         } else {
-            Q.a = tp_sound_speed<M, NSP>(*A.gas, Q);
+            Q.a = tp_sound_speed<M, NSP>(tp_gas(A), Q);
             double* P = A.Pout;
             P[P_RHO * qs + c] = Q.rho; P[P_VX * qs + c] = v[0]; P[P_VY * qs + c] = v[1]; P[P_VZ * qs + c] = v[2];
             P[P_U * qs + c] = Q.u; P[P_T * qs + c] = Q.T; P[P_P * qs + c] = Q.p; P[P_A * qs + c] = Q.a;
@@ -1167,7 +1161,7 @@ __global__ __launch_bounds__(64) void tp_boundary_face_kernel(TPArgs A)
     TPRef r[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) r[m] = tp_ref(A, i + (m - 2) * di, j + (m - 2) * dj, k + (m - 2) * dk);
-    const TPGas& g = *A.gas;
+    const TPGas& g = tp_gas(A);
     double F[5 + NSP];
 #pragma unroll
     for (int q = 0; q < 5 + NSP; ++q) F[q] = 0.0;
@@ -1338,7 +1332,7 @@ __global__ __launch_bounds__(128) void tp_extrap1_kernel(TPArgs A, int face)
         Q.T = dst[P_T * gs];
         Q.p = dst[P_P * gs];
         int fe = 0;
-        tp_update_thermo_from_rhou<MA, NSP>(*A.gas, Q, &fe);
+        tp_update_thermo_from_rhou<MA, NSP>(tp_gas(A), Q, &fe);
         const double vx = 2.0 * p1[P_VX * s1] - p2[P_VX * s2];
         const double vy = 2.0 * p1[P_VY * s1] - p2[P_VY * s2];
         const double vz = 2.0 * p1[P_VZ * s1] - p2[P_VZ * s2];
