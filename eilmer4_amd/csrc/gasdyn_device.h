@@ -166,11 +166,22 @@ __device__ __forceinline__ void interp_l2r2_scalar(const L2R2WT<typename M::R>& 
         sL = dv<M>(delLminus * del + ab(delLminus * del) + eps, delLminus * delLminus + del * del + eps);
         sR = dv<M>(del * delRplus + ab(del * delRplus) + eps, del * del + delRplus * delRplus + eps);
     }
-    qL = qL0 + sL * w.aL0 * (del * w.two_lenL0_plus_lenL1 + delLminus * w.lenR0);
-    qR = qR0 - sR * w.aR0 * (delRplus * w.lenL0 + del * w.two_lenR0_plus_lenR1);
+    R eL, eR;
+    if constexpr (M::kFast) {
+        // which product is fused into the sum is fixed here: left to the
+        // compiler it changed with the code around, and with it the FP32
+        // roundings of the mixed form
+        eL = fma(delLminus, w.lenR0, del * w.two_lenL0_plus_lenL1);
+        eR = fma(del, w.two_lenR0_plus_lenR1, delRplus * w.lenL0);
+    } else {
+        eL = del * w.two_lenL0_plus_lenL1 + delLminus * w.lenR0;
+        eR = delRplus * w.lenL0 + del * w.two_lenR0_plus_lenR1;
+    }
+    qL = qL0 + sL * w.aL0 * eL;
+    qR = qR0 - sR * w.aR0 * eR;
     if (extrema_clipping) {
-        qL = clip_to_limits(qL, qL0, qR0);
-        qR = clip_to_limits(qR, qL0, qR0);
+        qL = clip_limits<M>(qL, qL0, qR0);
+        qR = clip_limits<M>(qR, qL0, qR0);
     }
 }
 
