@@ -526,6 +526,7 @@ int stage_args_for(const BlockH& b, int stage, double dt, unsigned int* counters
     const int nk = A.nk;
     A.tiles_x = (b.ni + TILE_X - 1) / TILE_X;
     A.tiles_y = (b.nj + TILE_Y - 1) / TILE_Y;
+    A.sd_kc = e4::shock_detect_planes(A.ni, A.nj, nk);
     grid = dim3(A.tiles_x, A.tiles_y, (nk + A.kchunk - 1) / A.kchunk);
     return E4HIP_OK;
 }
@@ -858,6 +859,15 @@ int launch_stage_batch(const std::vector<const BlockH*>& blks, const std::vector
     }
     const size_t nstage_wg = map.size();
     map.insert(map.end(), bmap.begin(), bmap.end());
+    // and the detector's (a tuning run leaves the indicators alone)
+    const size_t ndetect0 = map.size();
+    if (flux_detects_shocks(cfg.flux_calculator) && force_chunks <= 0) {
+        for (int e = 0; e < n; ++e) {
+            args[e].swg0 = (int)(map.size() - ndetect0);
+            map.insert(map.end(), e4::shock_detect_workgroups(args[e], blks[e]->dims), e);
+        }
+    }
+    const int ndetect = (int)(map.size() - ndetect0);
     char *ad = nullptr, *md = nullptr;
     int rc = stage_batch_buffers(g_state.batch, batch_slot(set, stage, blks[0]->dims), args.data(),
                                  sizeof(e4::StageArgs) * n, map.data(), sizeof(int) * map.size(), &ad, &md);
@@ -867,6 +877,18 @@ int launch_stage_batch(const std::vector<const BlockH*>& blks, const std::vector
     B.wg_entry = (const int*)md;
     const bool def = args[0].high_order && args[0].apply_limiter && args[0].extrema_clipping;
     const int flux = kernel_flux(cfg.flux_calculator);
+    if (ndetect > 0) {
+        // every block's detection reads its neighbours' states and writes its own
+        // indicators only, so it may run just before the batch's fluxes
+        e4::BatchArgs Bs{};
+        Bs.table = B.table;
+        Bs.wg_entry = (const int*)md + ndetect0;
+        if (cfg.precision_mode == E4HIP_PRECISION_FP64_EXACT)
+            e4::launch_shock_detect_batch_exact(Bs, ndetect, blks[0]->dims, g_state.stream);
+        else
+            e4::launch_shock_detect_batch_fast64(Bs, ndetect, blks[0]->dims, g_state.stream);
+        HIP_TRY(hipGetLastError());
+    }
     hipEvent_t ev = nullptr;
     prof_begin(&ev);
     int nwg = (int)nstage_wg;
@@ -2014,8 +2036,17 @@ static int enqueue_step(const int* blks, int nblk, double dt, int ns, unsigned i
                 BlockH& b = *get_block(blks[n]);
                 std::swap(b.S[0], b.S[1]);
             }
+            // (the blocks of a batched stage detect in one launch of that stage)
+            int nideal[2] = {0, 0};
             for (int n = 0; n < nblk; ++n) {
-                rc = launch_shock_detect(*get_block(blks[n]), stage, dt);
+                const BlockH& b = *get_block(blks[n]);
+                if (!b.has_P()) ++nideal[b.dims - 2];
+            }
+            for (int n = 0; n < nblk; ++n) {
+                const BlockH& b = *get_block(blks[n]);
+                if (!b.has_P() && batch && g_state.cfg.batch_blocks && nideal[b.dims - 2] >= g_state.batch_min_blocks)
+                    continue;
+                rc = launch_shock_detect(b, stage, dt);
                 if (rc) return rc;
             }
         }

@@ -101,6 +101,7 @@ struct StageArgs {
     int tiles_x, tiles_y;             // workgroup tiles along i and j
     int wg0;                          // first workgroup of this block in a batched launch
     int bwg0;                         // first workgroup of this block in a batched boundary-cell launch
+    int swg0, sd_kc;                  // the same of a batched shock-detector launch; its planes per workgroup
     // shock indicators (adaptive_hanel_ausmdv, hanel): S of this stage's
     // detection, Sprev of the previous one (what the ghost cells were filled
     // with), the connected blocks' Sprev; Snew is written by the detector
@@ -337,6 +338,8 @@ void launch_tp_stage_mixed(const TPArgs& A, hipStream_t stream, int flux);
 // mixed mode uses the fast64 detector (FP64 arithmetic)
 void launch_shock_detect_exact(const StageArgs& A, int dims, hipStream_t stream);
 void launch_shock_detect_fast64(const StageArgs& A, int dims, hipStream_t stream);
+void launch_shock_detect_batch_exact(const BatchArgs& B, int nwg, int dims, hipStream_t stream);
+void launch_shock_detect_batch_fast64(const BatchArgs& B, int nwg, int dims, hipStream_t stream);
 void launch_tp_shock_detect_exact(const TPArgs& A, hipStream_t stream);
 void launch_tp_shock_detect_fast64(const TPArgs& A, hipStream_t stream);
 void launch_tp_decode_exact(const TPArgs& A, const double* U, const double* Tguess, hipStream_t stream);
@@ -366,5 +369,23 @@ void launch_boundary_cells_mixed(const StageArgs& A, hipStream_t stream, int dim
 
 constexpr int TILE_X = 32;
 constexpr int TILE_Y = 8;
+
+// Tile of the ideal-gas shock detector: cells of a wave's row, rows of a workgroup.
+constexpr int SD_TX = 62, SD_TY = 8;
+
+// Planes per workgroup of the detector: short enough for about 1024 workgroups
+// (two rounds of what the chip holds; 512 and 2048 measured 3-8 % slower), long enough that the plane read twice at each end
+// of a chunk does not count.
+inline int shock_detect_planes(int ni, int nj, int nk)
+{
+    const long cols = (long)((ni + SD_TX - 1) / SD_TX) * ((nj + SD_TY - 1) / SD_TY);
+    const long kc = cols * nk / 1024;
+    return (int)(kc < 4 ? 4 : (kc > 16 ? 16 : kc));
+}
+inline int shock_detect_workgroups(const StageArgs& A, int dims)
+{
+    const int kz = (dims == 3) ? (A.nk + A.sd_kc - 1) / A.sd_kc : 1;
+    return ((A.ni + SD_TX - 1) / SD_TX) * ((A.nj + SD_TY - 1) / SD_TY) * kz;
+}
 
 } // namespace e4

@@ -39,4 +39,9 @@ void launch_shock_detect_exact(const StageArgs& A, int dims, hipStream_t stream)
     launch_shock_detect_mode<ModeExact>(A, dims, stream);
 }
 
+void launch_shock_detect_batch_exact(const BatchArgs& B, int nwg, int dims, hipStream_t stream)
+{
+    launch_shock_detect_batch_mode<ModeExact>(B, nwg, dims, stream);
+}
+
 } // namespace e4

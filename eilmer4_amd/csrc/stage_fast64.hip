@@ -39,4 +39,9 @@ void launch_shock_detect_fast64(const StageArgs& A, int dims, hipStream_t stream
     launch_shock_detect_mode<ModeFast64>(A, dims, stream);
 }
 
+void launch_shock_detect_batch_fast64(const BatchArgs& B, int nwg, int dims, hipStream_t stream)
+{
+    launch_shock_detect_batch_mode<ModeFast64>(B, nwg, dims, stream);
+}
+
 } // namespace e4

@@ -1191,103 +1191,223 @@ void launch_stage_mode(const StageArgs& A, dim3 grid, hipStream_t stream, int di
 // (u_n,right - u_n,left) / min(a_left, a_right) < compression tolerance (the
 // face normal of this axis-aligned grid is a unit axis); a cell is one when
 // any of its faces is.  Ghost neighbours are the ghost-cell effects' states.
+// Velocity and sound speed of a cell for the detector: q is the sound speed in
+// ModeExact; in the fast modes its square, which the face test compares with
+// the squared velocity jump (no square root, no division).
+struct SdState {
+    double v0, v1, v2, q;
+};
+
 template <class M>
-__device__ __forceinline__ Prim prim_at(KArgs A, int i, int j, int k)
+__device__ __forceinline__ SdState sd_decode(const double U[5], const IdealGas& g)
 {
-    if (i >= 0 && i < A->ni && j >= 0 && j < A->nj && k >= 0 && k < A->nk)
-        return load_decode<M>(A, cell_index(A, i, j, k));
-    return fetch_ghost<M, false, true>(A, i, j, k);
+    if constexpr (!M::kFast) {
+        const Prim P = decode_ideal<M>(U[0], U[1], U[2], U[3], U[4], g);
+        return SdState{P.v0, P.v1, P.v2, P.a};
+    } else {
+        const double dinv = dv<ModeFast64>(1.0, U[0]);
+        SdState s{U[1] * dinv, U[2] * dinv, U[3] * dinv, 0.0};
+        const double u = U[4] * dinv - 0.5 * (s.v0 * s.v0 + s.v1 * s.v1 + s.v2 * s.v2);
+        s.q = g.gammaR * (u * g.Cvinv);
+        return s;
+    }
 }
 
-__device__ __forceinline__ double prim_vel(const Prim& P, int d) { return d == 0 ? P.v0 : (d == 1 ? P.v1 : P.v2); }
-
-// A workgroup owns a 32 x 8 column of cells and marches a chunk of k-planes:
-// each plane, with a one-cell ring in i and j, is decoded once into LDS
-// (velocity and sound speed; double-buffered so that plane k+1 loads while
-// plane k is tested); the k-direction neighbours come from the next plane
-// and from the thread's previous cell.
-constexpr int SD_TX = 32, SD_TY = 8, SD_KC = 16;
-
-template <class M, int DIMS>
-__global__ __launch_bounds__(256) void shock_detect_kernel(StageArgs)
+// Whether a jump d of normal velocity is a shock point against the smaller
+// sound speed m (or its square): d / a < tol.
+template <class M>
+__device__ __forceinline__ bool sd_hit(double d, double m, double tol)
 {
-    using MD = typename std::conditional<M::kFast, ModeFast64, ModeExact>::type;
-    constexpr int TX = SD_TX, TY = SD_TY, PX = TX + 2, PY = TY + 2, PL = PX * PY;
-    __shared__ double sv[2][4][PL];          // vx, vy, vz, a of a plane and its ring
-    KArgs A = kargs();
-    if (stage_aborted(A->abort_prev)) return;
-    const int i0 = blockIdx.x * TX, j0 = blockIdx.y * TY;
-    const int k0 = (DIMS == 3) ? blockIdx.z * SD_KC : 0;
-    const int k1 = (DIMS == 3) ? min(k0 + SD_KC, A->nk) : 1;
-    const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
-    const int i = i0 + tx, j = j0 + ty;
-    const bool own = i < A->ni && j < A->nj;
-    const int h = (ty + 1) * PX + (tx + 1);
-    auto load_plane = [&](int buf, int k) {
-        for (int t = threadIdx.x; t < PL; t += blockDim.x) {
-            const int hx = t % PX, hy = t / PX;
-            // ring corners are never read; positions outside in two
-            // directions give a dummy state
-            const Prim P = prim_at<M>(A, i0 + hx - 1, j0 + hy - 1, k);
-            sv[buf][0][t] = P.v0; sv[buf][1][t] = P.v1; sv[buf][2][t] = P.v2; sv[buf][3][t] = P.a;
-        }
-    };
-    const double tol = A->compression_tol;
-    auto face = [&](double uL, double aL, double uR, double aR) {
-        const double a_min = (aL < aR) ? aL : aR;
-        return dv<MD>(uR - uL, a_min) < tol;
-    };
-    double vz_below = 0.0, a_below = 1.0;
-    if constexpr (DIMS == 3) {
-        if (own) {
-            const Prim P = prim_at<M>(A, i, j, k0 - 1);
-            vz_below = P.v2;
-            a_below = P.a;
-        }
+    if constexpr (!M::kFast) return dv<M>(d, m) < tol;
+    else if (tol < 0.0) return d < 0.0 && m > 0.0 && d * d > (tol * tol) * m;
+    else return d < 0.0 || d * d < (tol * tol) * m;
+}
+
+__device__ __forceinline__ double sd_min(double aL, double aR) { return (aL < aR) ? aL : aR; }
+
+// The value of the lane above (lane 63: 0): two moves between neighbouring lanes.
+__device__ __forceinline__ double lane_above(double x)
+{
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+    const unsigned int lo = (unsigned int)__builtin_amdgcn_update_dpp(0, (int)(unsigned int)b, 0x130, 0xf, 0xf, true);
+    const unsigned int hi = (unsigned int)__builtin_amdgcn_update_dpp(0, (int)(unsigned int)(b >> 32), 0x130, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// Where a line's position outside the block (-1, or n) takes its state from, for
+// the ghost kinds that copy a cell of the block: the cell's position on the line;
+// *flip when a slip wall mirrors it, *special for the other kinds (inflow,
+// connected, stored), whose position is then 0.
+__device__ __forceinline__ int sd_source(int type, bool plus, int n, bool* flip, bool* special)
+{
+    *special = type == BC_INFLOW || type == BC_CONNECTED || type == BC_INFLOW_PROFILE || type == BC_EXTRAPOLATE_1;
+    *flip = type == BC_SLIP_WALL || type == BC_SLIP_WALL_1;
+    if (*special) return 0;
+    return (plus != (type == BC_PERIODIC)) ? n - 1 : 0;
+}
+
+// A wave owns a row of SD_TX cells in i, one lane beyond it on either side, and
+// marches sd_kc planes in k; a workgroup is SD_TY such rows in j.  A lane
+// decodes its own column once per plane and keeps it for the k faces; the i
+// neighbour comes from the next lane, the j neighbours from the other waves
+// through LDS (double-buffered: one barrier a plane), the rows beyond the
+// workgroup from memory.  Positions outside the block that copy one of its
+// cells are loads of that cell like any other; the other ghosts go through one
+// rare branch per plane.  The next plane's values are loaded while this one is
+// tested.  Bound by the latency of those loads (16 waves a compute unit fit);
+// loading two planes ahead did not help.  Against a 32 x 8 tile whose planes
+// went through LDS whole, with two barriers, divisions and square roots: 128^3
+// 88 -> 47 us, 256^3 370 -> 238 us (2.9 TB/s); joined 2D blocks in one launch
+// instead of one each.
+template <class M, int DIMS, bool BATCH>
+__global__ __launch_bounds__(64 * SD_TY) void shock_detect_kernel(
+    typename std::conditional<BATCH, BatchArgs, StageArgs>::type)
+{
+    KArgs A;
+    int wg = (int)blockIdx.x;
+    if constexpr (BATCH) {
+        A = kargs_entry(batch_entry());
+        wg -= A->swg0;
+    } else {
+        A = kargs();
     }
-    load_plane(0, k0);
-    int buf = 0;
-    for (int k = k0; k < k1; ++k) {
-        if constexpr (DIMS == 3) load_plane(buf ^ 1, k + 1);
-        __syncthreads();
-        if (own) {
-            const double (*c)[PL] = sv[buf];
+    if (stage_aborted(A->abort_prev)) return;
+    const int ni = A->ni, nj = A->nj, nk = (DIMS == 3) ? A->nk : 1;
+    const int tiles_x = (ni + SD_TX - 1) / SD_TX, tiles_y = (nj + SD_TY - 1) / SD_TY;
+    const int bx = wg % tiles_x, by = (wg / tiles_x) % tiles_y, bz = wg / (tiles_x * tiles_y);
+    const int lane = (int)(threadIdx.x & 63u);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int j = by * SD_TY + w;
+    const bool row = j < nj;                           // (waves without a row keep to the barriers)
+    const int k0 = (DIMS == 3) ? bz * A->sd_kc : 0;
+    const int k1 = (DIMS == 3) ? min(k0 + A->sd_kc, nk) : 1;
+    const int i = min(bx * SD_TX - 1 + lane, ni);      // lanes past the block repeat its last ghost
+    const bool own = row && i >= 0 && i < ni && lane >= 1 && lane <= SD_TX;
+    const double tol = A->compression_tol;
+    const int ng = A->noghost;
+    // the lane's column: a cell of the block, or what an i ghost copies
+    bool iflip = false, ispecial = false;
+    int ic = i;
+    if (i < 0 || i >= ni) ic = sd_source(A->bc->type[i < 0 ? FACE_WEST : FACE_EAST], i >= ni, ni, &iflip, &ispecial);
+    // the rows below and above: another wave's, or loaded here
+    __shared__ double2 sJ[2][SD_TY][64];               // (v1, q) of the rows' current plane
+    const bool mload = row && (w == 0 || j == 0), pload = row && (w == SD_TY - 1 || j == nj - 1);
+    bool mflip = false, mspecial = false, pflip = false, pspecial = false;
+    int jm = j - 1, jp = j + 1;
+    if (jm < 0) jm = sd_source(A->bc->type[FACE_SOUTH], false, nj, &mflip, &mspecial);
+    if (jp >= nj) jp = sd_source(A->bc->type[FACE_NORTH], true, nj, &pflip, &pspecial);
+    const long qs = A->qs;
+    const double* __restrict__ U = A->Us;
+    auto load = [&](int jj, int kk, double r[5]) {
+        const unsigned int off = (((unsigned int)kk * nj + jj) * ni + ic) * 8u;
+#pragma unroll
+        for (int q = 0; q < 5; ++q) r[q] = *(const double*)((const char*)(U + q * qs) + off);
+    };
+    // plane kk of the lane's column, with what its k ghosts copy
+    auto load_column = [&](int kk, double r[5], bool* flip, bool* special) {
+        *flip = false;
+        *special = false;
+        if (DIMS == 3 && (kk < 0 || kk >= nk))
+            kk = sd_source(A->bc->type[kk < 0 ? FACE_BOTTOM : FACE_TOP], kk >= nk, nk, flip, special);
+        load(row ? j : nj - 1, kk, r);
+    };
+    double rc[5], rm[5], rp[5];
+    bool cflip, cspecial;
+    SdState C{}, N;
+    bool below = false;                                // the face under the current plane is a shock point
+    constexpr int LEAD = (DIMS == 3) ? 2 : 1;          // turns that only fetch planes k0 - 1 and k0
+    load_column(k0 - LEAD + 1, rc, &cflip, &cspecial);
+    for (int k = k0 - LEAD; k < k1; ++k) {
+        const bool test = k >= k0;
+        const IdealGas gas = A->gas;
+        SdState Jm, Jp;
+        N = sd_decode<M>(rc, gas);
+        if (iflip) N.v0 = -N.v0;
+        if (cflip) N.v2 = -N.v2;
+        bool nspecial = ispecial || cspecial;
+        if (DIMS == 2 && k == 0) nspecial = false;     // (no plane follows)
+        if (test) {
+            __syncthreads();                           // the rows' (v1, q) of this plane are in sJ
+            if (mload) {
+                Jm = sd_decode<M>(rm, gas);
+                if (mflip) Jm.v1 = -Jm.v1;
+            } else {
+                const double2 x = sJ[k & 1][w > 0 ? w - 1 : 0][lane];
+                Jm.v1 = x.x; Jm.q = x.y;
+            }
+            if (pload) {
+                Jp = sd_decode<M>(rp, gas);
+                if (pflip) Jp.v1 = -Jp.v1;
+            } else {
+                const double2 x = sJ[k & 1][w < SD_TY - 1 ? w + 1 : w][lane];
+                Jp.v1 = x.x; Jp.q = x.y;
+            }
+        }
+        if (row && __ballot(nspecial || (test && (mspecial || pspecial))) != 0) {
+#pragma nounroll
+            for (int g = 0; g < 3; ++g) {
+                // the next plane's cell (in i or k outside the block), the rows below and above
+                if (!(g == 0 ? nspecial : (test && i >= 0 && i < ni && (g == 1 ? mspecial : pspecial)))) continue;
+                const Prim P = fetch_ghost<M, false, true>(A, i, (g == 0) ? j : (g == 1) ? j - 1 : j + 1,
+                                                           (g == 0) ? k + 1 : k);
+                const SdState G{P.v0, P.v1, P.v2, M::kFast ? P.a * P.a : P.a};
+                if (g == 0) N = G;
+                else if (g == 1) Jm = G;
+                else Jp = G;
+            }
+        }
+        // the loads of the next turn
+        if (DIMS == 3 && k + 1 < k1) load_column(k + 2, rc, &cflip, &cspecial);
+        if (k + 1 >= k0 && k + 1 < k1) {
+            if (mload) load(jm, k + 1, rm);
+            if (pload) load(jp, k + 1, rp);
+        }
+        bool above = false;
+        if constexpr (DIMS == 3) {
             // a boundary face without ghost data has the cell on one side only
             // (shockdetectors.d:39-54): its velocity towards the wall
-            const int ng = A->noghost;
-            const double a0 = c[3][h];
-            auto minus_face = [&](bool wall, double uL, double aL, double u0) {
-                return wall ? dv<MD>(u0, a0) < tol : face(uL, aL, u0, a0);
-            };
-            auto plus_face = [&](bool wall, double u0, double uR, double aR) {
-                return wall ? dv<MD>(-u0, a0) < tol : face(u0, a0, uR, aR);
-            };
-            bool S = minus_face(i == 0 && (ng & (1 << FACE_WEST)), c[0][h - 1], c[3][h - 1], c[0][h]) ||
-                     plus_face(i == A->ni - 1 && (ng & (1 << FACE_EAST)), c[0][h], c[0][h + 1], c[3][h + 1]) ||
-                     minus_face(j == 0 && (ng & (1 << FACE_SOUTH)), c[1][h - PX], c[3][h - PX], c[1][h]) ||
-                     plus_face(j == A->nj - 1 && (ng & (1 << FACE_NORTH)), c[1][h], c[1][h + PX], c[3][h + PX]);
-            if constexpr (DIMS == 3) {
-                const double (*n)[PL] = sv[buf ^ 1];
-                S = S || minus_face(k == 0 && (ng & (1 << FACE_BOTTOM)), vz_below, a_below, c[2][h]) ||
-                    plus_face(k == A->nk - 1 && (ng & (1 << FACE_TOP)), c[2][h], n[2][h], n[3][h]);
-                vz_below = c[2][h];
-                a_below = c[3][h];
-            }
-            A->Snew[cell_index(A, i, j, k)] = S ? 1 : 0;
+            if (k == nk - 1 && (ng & (1 << FACE_TOP))) above = sd_hit<M>(-C.v2, C.q, tol);
+            else if (k == -1 && (ng & (1 << FACE_BOTTOM))) above = sd_hit<M>(N.v2, N.q, tol);
+            else above = sd_hit<M>(N.v2 - C.v2, sd_min(C.q, N.q), tol);
         }
-        __syncthreads();
-        buf ^= 1;
+        if (test) {
+            const double vR = lane_above(C.v0), qR = lane_above(C.q);
+            bool e = (i == ni - 1 && (ng & (1 << FACE_EAST))) ? sd_hit<M>(-C.v0, C.q, tol)
+                                                             : sd_hit<M>(vR - C.v0, sd_min(C.q, qR), tol);
+            if (i < 0 && (ng & (1 << FACE_WEST))) e = false;
+            const unsigned long long em = __ballot(e);
+            bool S = e || (lane > 0 && ((em >> (lane - 1)) & 1ull));
+            if (i == 0 && (ng & (1 << FACE_WEST))) S = S || sd_hit<M>(C.v0, C.q, tol);
+            S = S || ((j == 0 && (ng & (1 << FACE_SOUTH))) ? sd_hit<M>(C.v1, C.q, tol)
+                                                          : sd_hit<M>(C.v1 - Jm.v1, sd_min(Jm.q, C.q), tol));
+            S = S || ((j == nj - 1 && (ng & (1 << FACE_NORTH))) ? sd_hit<M>(-C.v1, C.q, tol)
+                                                               : sd_hit<M>(Jp.v1 - C.v1, sd_min(C.q, Jp.q), tol));
+            if constexpr (DIMS == 3) S = S || below || above;
+            if (own) A->Snew[((long)k * nj + j) * ni + i] = S ? 1 : 0;
+        }
+        below = above;
+        C = N;
+        if (k + 1 >= k0 && k + 1 < k1) sJ[(k + 1) & 1][w][lane] = make_double2(C.v1, C.q);
     }
 }
 
 template <class M>
 void launch_shock_detect_mode(const StageArgs& A, int dims, hipStream_t stream)
 {
-    const dim3 block(SD_TX * SD_TY);
-    const dim3 grid((A.ni + SD_TX - 1) / SD_TX, (A.nj + SD_TY - 1) / SD_TY,
-                    (dims == 3) ? (A.nk + SD_KC - 1) / SD_KC : 1);
-    if (dims == 3) hipLaunchKernelGGL((shock_detect_kernel<M, 3>), grid, block, 0, stream, A);
-    else hipLaunchKernelGGL((shock_detect_kernel<M, 2>), grid, block, 0, stream, A);
+    const dim3 block(64 * SD_TY), grid((unsigned)shock_detect_workgroups(A, dims));
+    if (dims == 3) hipLaunchKernelGGL((shock_detect_kernel<M, 3, false>), grid, block, 0, stream, A);
+    else hipLaunchKernelGGL((shock_detect_kernel<M, 2, false>), grid, block, 0, stream, A);
+}
+
+// one launch over the blocks of a batched stage, each workgroup mapped to its
+// block by B.wg_entry (swg0: the block's first workgroup)
+template <class M>
+void launch_shock_detect_batch_mode(const BatchArgs& B, int nwg, int dims, hipStream_t stream)
+{
+    if (nwg <= 0) return;
+    const dim3 block(64 * SD_TY), grid((unsigned)nwg);
+    if (dims == 3) hipLaunchKernelGGL((shock_detect_kernel<M, 3, true>), grid, block, 0, stream, B);
+    else hipLaunchKernelGGL((shock_detect_kernel<M, 2, true>), grid, block, 0, stream, B);
 }
 
 } // namespace e4
