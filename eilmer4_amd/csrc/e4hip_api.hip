@@ -123,6 +123,8 @@ constexpr int ABORT_STRIDE = 32;
 // pointers per block in a step's snapshot (U[4], d[2], P[4], S[2])
 constexpr int PTRS_PER_BLOCK = 12;
 
+constexpr int CFL_BLOCKS = 128;                // blocks whose CFL signals e4hip_determine_dt reads back at a time
+
 struct State {
     bool init = false;
     int device = 0;
@@ -132,8 +134,9 @@ struct State {
     unsigned int* counters = nullptr;          // per-stage counters, e4::COUNTER_SLOT uints per block-stage slot
     unsigned int* counters_host = nullptr;     // pinned host copy the step reads the flags and counters back into
     unsigned int* step_abort = nullptr;        // abort flags of the step being enqueued
-    unsigned long long* smax = nullptr;
-    double* last_signal = nullptr;
+    unsigned long long* signals = nullptr;      // e4hip_determine_dt: per block its largest CFL signal (bit
+                                               // pattern) and its last cell's signal, CFL_BLOCKS pairs
+    unsigned long long* signals_host = nullptr; // their pinned host copy
     int counter_slots = 0;
     std::vector<GasModelH> gases;
     BatchBuffers batch;
@@ -1248,8 +1251,8 @@ int e4hip_init(int device)
         scratch_dev[device] = (unsigned long long*)p;
     }
     HIP_TRY(hipStreamCreateWithFlags(&g_state.stream, hipStreamNonBlocking));
-    HIP_TRY(hipMalloc(&g_state.smax, sizeof(unsigned long long)));
-    HIP_TRY(hipMalloc(&g_state.last_signal, sizeof(double)));
+    HIP_TRY(hipMalloc(&g_state.signals, sizeof(unsigned long long) * 2 * CFL_BLOCKS));
+    HIP_TRY(hipHostMalloc(&g_state.signals_host, sizeof(unsigned long long) * 2 * CFL_BLOCKS));
     HIP_TRY(hipMalloc(&g_state.queue, 2 * sizeof(unsigned int)));
     HIP_TRY(hipMemset(g_state.queue, 0, 2 * sizeof(unsigned int)));
     HIP_TRY(hipMalloc(&g_state.stats, sizeof(unsigned long long) * e4::STAT_LANES * e4::STAT_STRIDE));
@@ -1285,11 +1288,11 @@ int e4hip_finalize(void)
         if (bb->map_dev) { HIP_TRY(hipFree(bb->map_dev)); HIP_TRY(hipHostFree(bb->map_host)); }
         *bb = BatchBuffers();
     }
-    if (g_state.smax) HIP_TRY(hipFree(g_state.smax));
-    if (g_state.last_signal) HIP_TRY(hipFree(g_state.last_signal));
+    if (g_state.signals) HIP_TRY(hipFree(g_state.signals));
+    if (g_state.signals_host) HIP_TRY(hipHostFree(g_state.signals_host));
     if (g_state.queue) HIP_TRY(hipFree(g_state.queue));
     if (g_state.stats) HIP_TRY(hipFree(g_state.stats));
-    g_state.counters = nullptr; g_state.smax = nullptr; g_state.last_signal = nullptr; g_state.queue = nullptr;
+    g_state.counters = nullptr; g_state.signals = nullptr; g_state.signals_host = nullptr; g_state.queue = nullptr;
     g_state.counter_slots = 0;
     HIP_TRY(hipStreamDestroy(g_state.stream));
     g_state.stream = nullptr;
@@ -2369,22 +2372,29 @@ int e4hip_determine_dt(const int* blks, int nblk, double dt_current, double cfl_
     if (!g_state.init) return fail(E4HIP_ERR_NOT_INIT, "e4hip_init not called");
     if (!blks || nblk <= 0 || !dt_allow_out || !cfl_max_out) return fail(E4HIP_ERR_ARG, "bad arguments");
     double dt_allow_all = 1.7976931348623157e308, cfl_max_all = 0.0;
-    for (int n = 0; n < nblk; ++n) {
-        BlockH* b = get_block(blks[n]);
-        if (!b) return fail(E4HIP_ERR_HANDLE, "unknown block %d", blks[n]);
-        hipLaunchKernelGGL(e4::reset_counters_kernel, dim3(1), dim3(64), 0, g_state.stream, g_state.counters, 0,
-                           g_state.smax);
-        int rc = enqueue_cfl(*b, g_state.smax, g_state.last_signal);
-        if (rc) return rc;
-        unsigned long long bits = 0;
-        double last = 0.0;
-        HIP_TRY(hipMemcpyAsync(&bits, g_state.smax, sizeof(bits), hipMemcpyDeviceToHost, g_state.stream));
-        HIP_TRY(hipMemcpyAsync(&last, g_state.last_signal, sizeof(last), hipMemcpyDeviceToHost, g_state.stream));
+    for (int n = 0; n < nblk; ++n)
+        if (!get_block(blks[n])) return fail(E4HIP_ERR_HANDLE, "unknown block %d", blks[n]);
+    // the blocks' signals side by side, cleared, reduced and read back
+    // together: one wait for up to CFL_BLOCKS blocks instead of one (and two
+    // copies) for each
+    for (int n0 = 0; n0 < nblk; n0 += CFL_BLOCKS) {
+        const int m = std::min(CFL_BLOCKS, nblk - n0);
+        hipLaunchKernelGGL(noalloc_clear_kernel, dim3(1), dim3(256), 0, g_state.stream, g_state.signals, 2 * m);
+        for (int n = 0; n < m; ++n) {
+            unsigned long long* sp = g_state.signals + 2 * n;
+            int rc = enqueue_cfl(*get_block(blks[n0 + n]), sp, (double*)(sp + 1));
+            if (rc) return rc;
+        }
+        HIP_TRY(hipMemcpyAsync(g_state.signals_host, g_state.signals, sizeof(unsigned long long) * 2 * m,
+                               hipMemcpyDeviceToHost, g_state.stream));
         HIP_TRY(hipStreamSynchronize(g_state.stream));
-        double dt_allow, cfl_max;
-        block_dt(bits, last, dt_current, cfl_value, check_cfl, dt_allow, cfl_max);
-        dt_allow_all = fmin(dt_allow_all, dt_allow);
-        cfl_max_all = fmax(cfl_max_all, cfl_max);
+        for (int n = 0; n < m; ++n) {
+            double last, dt_allow, cfl_max;
+            memcpy(&last, &g_state.signals_host[2 * n + 1], sizeof(last));
+            block_dt(g_state.signals_host[2 * n], last, dt_current, cfl_value, check_cfl, dt_allow, cfl_max);
+            dt_allow_all = fmin(dt_allow_all, dt_allow);
+            cfl_max_all = fmax(cfl_max_all, cfl_max);
+        }
     }
     *dt_allow_out = dt_allow_all;
     *cfl_max_out = cfl_max_all;
