@@ -287,6 +287,8 @@ bool l2r2_uniform(double len, e4::L2R2U& u)
     u.a = w.aL0;
     u.len = w.lenR0;
     u.len3 = w.two_lenL0_plus_lenL1;
+    u.wt = u.a * u.len * u.c;
+    u.epsl = 1.0e-12 / (u.c * u.c);
     return w.two_over_lenR0_plus_lenL0 == u.c && w.two_over_lenR1_plus_lenR0 == u.c && w.aR0 == u.a &&
            w.lenL0 == u.len && w.two_lenR0_plus_lenR1 == u.len3;
 }
@@ -1328,6 +1330,7 @@ int e4hip_gas_ideal(double mMass, double gamma, int* gm)
     g.ideal.Cvinv = 1.0 / g.ideal.Cv;
     g.ideal.gammaR = gamma * g.ideal.Rgas;
     g.ideal.CpCv = (g.ideal.Rgas * gamma / (gamma - 1.0)) / g.ideal.Cv;   // gas_model.d:162, ideal_gas.d:68
+    g.ideal.RonCv = g.ideal.Rgas * g.ideal.Cvinv;
     g_state.gases.push_back(g);
     *gm = (int)g_state.gases.size() - 1;
     return E4HIP_OK;

@@ -251,6 +251,26 @@ __device__ __forceinline__ void interp_l2r2_cell(const L2R2UT<typename M::R>& w,
                                                  typename M::R qp, typename M::R& qLp, typename M::R& qRm)
 {
     using R = typename M::R;
+    if constexpr (std::is_same<M, ModeFast64>::value) {
+        // the same in the differences themselves: with d = e c the limiter's
+        // c^2 cancels but for eps, and len3 = 3 len, so both corrections are
+        // s wt times (3 e1 + e0) and (3 e0 + e1); 24 FP64 operations and a
+        // reciprocal seed instead of 34 and one
+        const double e0 = q0 - qm, e1 = qp - q0;
+        double t = w.wt;
+        if (apply_limiter) {
+            const double den = fma(e0, e0, fma(e1, e1, w.epsl));
+            const double num = fma(e0, e1, fabs(e0 * e1) + w.epsl);
+            t = num * rcp_full(den) * w.wt;
+        }
+        qLp = fma(t, fma(3.0, e1, e0), q0);
+        qRm = fma(-t, fma(3.0, e0, e1), q0);
+        if (extrema_clipping) {
+            qLp = min_raw(max_raw(qLp, min_raw(q0, qp)), max_raw(q0, qp));
+            qRm = min_raw(max_raw(qRm, min_raw(qm, q0)), max_raw(qm, q0));
+        }
+        return;
+    }
     const R eps = R(1.0e-12);   // onedinterp.d:22
     R dm = (q0 - qm) * w.c;
     R dp = (qp - q0) * w.c;
@@ -333,7 +353,12 @@ __device__ __forceinline__ void side_flux(const SideT<typename M::R>& L, const S
     R TR = Rf.u * g.Cvinv;
     Lf.T = TL;
     Rf.T = TR;
-    if constexpr (M::kFast) {
+    if constexpr (std::is_same<M, ModeFast64>::value) {
+        Lf.RT = g.RonCv * Lf.u;
+        Rf.RT = g.RonCv * Rf.u;
+        Lf.p = Lf.rho * Lf.RT;
+        Rf.p = Rf.rho * Rf.RT;
+    } else if constexpr (M::kFast) {
         Lf.RT = g.Rgas * TL;
         Rf.RT = g.Rgas * TR;
         Lf.p = Lf.rho * Lf.RT;
