@@ -19,12 +19,23 @@
 //      limiter evaluation per scalar: on the uniform grid the van Albada
 //      factor of both is the same expression of the same two differences, so
 //      the results are those of the per-face evaluation of
-//      onedinterp.d:136-162, bit for bit.  Right states go to LDS; the
-//      k-direction stencil lives in a three-plane register queue;
-//   3. every cell evaluates the flux of its plus faces (i, j from LDS, k from
-//      registers); fluxes of the tile's west and south faces are extra items;
-//   4. flux divergence, stage update, decode check and the write of the new
+//      onedinterp.d:136-162, bit for bit (the plain FP64 form regroups them
+//      to save operations).  Right states go to LDS; the k-direction stencil
+//      lives in registers;
+//   3. every cell evaluates the flux of its east and north faces from LDS;
+//      fluxes of the tile's west and south faces are extra items;
+//   4. every cell evaluates the flux of its top face from registers (the mixed
+//      form a plane ahead, after 5);
+//   5. flux divergence, stage update, decode check and the write of the new
 //      state happen in registers.
+//
+// The FP64 form is bound by FP64 issue: a cell takes about 1100 vector
+// instructions and the kernel keeps the units three quarters busy at the 12 waves a
+// compute unit that 168 registers and 48 KB of LDS allow; a spill or a lower
+// occupancy costs more than the operations it saves.  256^3 ausmdv, one stage:
+// 1.252 ms; 1.065 with the shorter reconstruction and flux; 1.015 with the
+// k direction within the iteration, which ended the spills; 0.994 with the halo
+// cells loaded ahead.
 #pragma once
 #include "stage_args.h"
 
@@ -506,6 +517,37 @@ template <> struct StageOccupancy<ModeMixed> { static constexpr int waves = E4_S
 
 // DEF: the default reconstruction (order 2, limiter, extrema clipping) fixed
 // at compile time; otherwise the three options are read from the arguments.
+// A thread's halo cell of the tile, the same position in every plane: the offset
+// within a plane of the cell it reads -- the cell itself, or the one that a wall,
+// extrapolation or periodic ghost copies -- with flags in the upper bits, or
+// HALO_FETCH (an inflow or connected ghost, resolved by fetch) or HALO_NONE (a
+// position no face reads).  The same mapping as fetch_ghost's.
+enum : unsigned int { HALO_FLIP0 = 1u << 28, HALO_FLIP1 = 1u << 29, HALO_GHOST = 1u << 30, HALO_NONE = 0xfffffffeu,
+                      HALO_FETCH = 0xffffffffu };
+
+__device__ __forceinline__ unsigned int halo_position(KArgs A, int i, int j)
+{
+    const int ni = A->ni, nj = A->nj;
+    const bool in_i = i >= 0 && i < ni, in_j = j >= 0 && j < nj;
+    if ((long)ni * nj >= (long)HALO_FLIP0) return HALO_FETCH;
+    if (in_i && in_j) return (unsigned int)(j * ni + i);
+    if (!in_i && !in_j) return HALO_NONE;
+    const int idx = in_j ? i : j, n = in_j ? ni : nj;
+    const bool plus = idx >= n;
+    const int layer = plus ? idx - n + 1 : -idx;
+    if (layer > 2) return HALO_NONE;
+    const int face = in_j ? (plus ? FACE_EAST : FACE_WEST) : (plus ? FACE_NORTH : FACE_SOUTH);
+    const int type = A->bc->type[face];
+    if (type == BC_INFLOW || type == BC_CONNECTED) return HALO_FETCH;
+    int src;
+    if (type == BC_EXTRAPOLATE || type == BC_OUTFLOW_SIMPLE_FLUX) src = plus ? n - 1 : 0;
+    else if (type == BC_PERIODIC) src = plus ? layer - 1 : n - layer;
+    else src = plus ? n - layer : layer - 1;
+    unsigned int h = (unsigned int)(in_j ? j * ni + src : src * ni + i) | HALO_GHOST;
+    if (type == BC_SLIP_WALL || type == BC_SLIP_WALL_1) h |= in_j ? HALO_FLIP0 : HALO_FLIP1;
+    return h;
+}
+
 // One tile of the stage: with BATCH, tile wg of the launch's tile list (the
 // workgroup's own index, or the one it took from the work queue); without,
 // the workgroup's grid position.
@@ -522,8 +564,7 @@ __device__ __forceinline__ void stage_tile(int wg)
     constexpr int NSI = (TX + 1) * TY;       // i-face slots: face fc (0..TX) of row r is r*(TX+1)+fc
     constexpr int NSJ = TX * (TY + 1);       // j-face slots: face fr (0..TY) of column c is fr*TX+c
     constexpr int NHALO = 2 * (TX + TY);     // face states of halo cells
-    constexpr int NBND = TX + TY;            // west and south faces of the tile
-    static_assert(NHALO <= NT && NBND <= NT, "tile too narrow for its halo work");
+    static_assert(NHALO <= NT && TX <= 64 && 64 + TY <= NT, "tile too narrow for its halo work");
     // j-face frame
     constexpr int JN = 1, JT1 = (DIMS == 3) ? 2 : 0, JT2 = (DIMS == 3) ? 0 : 2;
     __shared__ R sP[6 * PLANE];              // rho, vx, vy, vz, u, a of plane k with halos
@@ -552,10 +593,16 @@ __device__ __forceinline__ void stage_tile(int wg)
     const bool clip = DEF || ap->extrema_clipping != 0;
 
     // k-direction register queue at the top of iteration k: own = plane k,
-    // qa = k+1, qb = k+2; LpC is the left state of the top face of cell k+1,
-    // Ft and Fb the fluxes of the own cell's top and bottom faces.  The
-    // k-direction work of the next plane is done at the end of an iteration,
-    // where the i/j face states are no longer live.
+    // qa = k+1; LpC is the left state of the own cell's top face (its sound
+    // speed is the own cell's), Fb the flux of its bottom face.  The FP64 forms
+    // evaluate the flux of the top face within the iteration, after the i and j
+    // fluxes, when their states are no longer live and the own state is read
+    // back from LDS: 21 values live through the i/j phases instead of 33, and no
+    // spill.  The mixed form, whose values are half as wide, is a plane ahead
+    // (KAHEAD): qb = k+2, LpC the left state of the top face of cell k+1, Ft the
+    // flux of the own cell's top face, and the next plane's work at the end of
+    // the iteration.
+    constexpr bool KAHEAD = std::is_same<M, ModeMixed>::value;
     PrimT<R> own, qa, qb;
     SideT<R> LpC;
     R Ft[5] = {R(0), R(0), R(0), R(0), R(0)}, Fb[5] = {R(0), R(0), R(0), R(0), R(0)};
@@ -566,13 +613,58 @@ __device__ __forceinline__ void stage_tile(int wg)
         PrimT<R> qm1 = fetch<M, SH>(ap, i, j, k0 - 1);
         own = fetch<M, SH>(ap, i, j, k0);
         qa = fetch<M, SH>(ap, i, j, k0 + 1);
-        qb = fetch<M, SH>(ap, i, j, k0 + 2);
+        if constexpr (KAHEAD) qb = fetch<M, SH>(ap, i, j, k0 + 2);
         SideT<R> Lbelow, Rdummy, Lown, Rown, Rabove;
         recon_cell<M>(wk, ho, lim, clip, qm2, qm1, own, Lbelow, Rdummy);
         recon_cell<M>(wk, ho, lim, clip, qm1, own, qa, Lown, Rown);
         if (own_ij) side_flux<M, FLUX, 2, 0, 1>(Lbelow, Rown, gR, Fb, shock_opt<R>(ap));
-        recon_cell<M>(wk, ho, lim, clip, own, qa, qb, LpC, Rabove);
-        if (own_ij) side_flux<M, FLUX, 2, 0, 1>(Lown, Rabove, gR, Ft, shock_opt<R>(ap));
+        LpC = Lown;
+        if constexpr (KAHEAD) {
+            recon_cell<M>(wk, ho, lim, clip, own, qa, qb, LpC, Rabove);
+            if (own_ij) side_flux<M, FLUX, 2, 0, 1>(Lown, Rabove, gR, Ft, shock_opt<R>(ap));
+        }
+    }
+
+    // The halo cell of plane k is loaded during the k-direction work of the plane
+    // before: its trip to memory stood at the top of every plane, ahead of a
+    // barrier.
+    constexpr int NHC = 4 * (TX + TY);
+    static_assert(NHC <= NT, "one halo cell per thread");
+    // 256^3 FP64 1.015 -> 0.994 ms.  (The mixed form gained nothing from it, nor
+    // either form from loading the update's old state before the barrier, and the
+    // exact form has no registers to spare.)
+    constexpr bool AHEAD = std::is_same<M, ModeFast64>::value;
+    unsigned int hpos = HALO_FETCH;
+    double hraw[5] = {1.0, 0.0, 0.0, 0.0, 1.0};
+    unsigned char hS = 0;
+    auto halo_ij = [&](int t, int& ii, int& jj) {
+        if (t < 4 * TY) {
+            int side = t / (2 * TY), rem = t % (2 * TY);
+            int col = rem / TY, row = rem % TY;
+            ii = side ? TX + 2 + col : col;
+            jj = row + 2;
+        } else {
+            int t2 = t - 4 * TY;
+            int side = t2 / (2 * TX), rem = t2 % (2 * TX);
+            int row = rem / TX, col = rem % TX;
+            jj = side ? TY + 2 + row : row;
+            ii = col + 2;
+        }
+    };
+    auto halo_load = [&](KArgs A, int k) {
+        if (hpos >= HALO_NONE) return;
+        const long qs = opaque_qs(A->qs);
+        const long c = (long)k * A->ni * A->nj + (hpos & (HALO_FLIP0 - 1u));
+        const double* p = A->Us + c;
+#pragma unroll
+        for (int q = 0; q < 5; ++q) hraw[q] = p[q * qs];
+        if (SH) hS = ((hpos & HALO_GHOST) ? A->Sprev : A->S)[c];
+    };
+    if (AHEAD && tid < NHC) {
+        int ii, jj;
+        halo_ij(tid, ii, jj);
+        hpos = halo_position(ap, i0 + ii - 2, j0 + jj - 2);
+        halo_load(ap, k0);
     }
 
     for (int k = k0; k < k1; ++k) {
@@ -584,12 +676,14 @@ __device__ __forceinline__ void stage_tile(int wg)
         const int ik = i0 + txk, jk = j0 + tyk;
         const bool own_k = (ik < ap->ni) && (jk < ap->nj);
         if constexpr (DIMS == 2) own = fetch<M, SH>(ap, ik, jk, 0);
-        // conserved state of plane k+3, loaded now and decoded at the end
+        // conserved state of plane k+2 (KAHEAD: k+3), loaded now and decoded for
+        // the k direction
+        constexpr int KRAW = KAHEAD ? 3 : 2;
         double raw[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        const bool raw_ok = (DIMS == 3) && own_k && (k + 1 < k1) && (k + 3 < ap->nk);
+        const bool raw_ok = (DIMS == 3) && own_k && (!KAHEAD || k + 1 < k1) && (k + KRAW < ap->nk);
         if (raw_ok) {
             const long qs = opaque_qs(ap->qs);
-            const double* p = ap->Us + cell_index(ap, ik, jk, k + 3);
+            const double* p = ap->Us + cell_index(ap, ik, jk, k + KRAW);
 #pragma unroll
             for (int q = 0; q < 5; ++q) raw[q] = p[q * qs];
         }
@@ -597,21 +691,21 @@ __device__ __forceinline__ void stage_tile(int wg)
         const int s0 = (tyk + 2) * PX + (txk + 2);
         sP[0 * PLANE + s0] = own.rho; sP[1 * PLANE + s0] = own.v0; sP[2 * PLANE + s0] = own.v1;
         sP[3 * PLANE + s0] = own.v2; sP[4 * PLANE + s0] = own.u; sP[5 * PLANE + s0] = own.a;
-        for (int t = tidk; t < 4 * (TX + TY); t += NT) {
+        if (tidk < NHC) {
             int ii, jj;
-            if (t < 4 * TY) {
-                int side = t / (2 * TY), rem = t % (2 * TY);
-                int col = rem / TY, row = rem % TY;
-                ii = side ? TX + 2 + col : col;
-                jj = row + 2;
+            halo_ij(tidk, ii, jj);
+            PrimT<R> h;
+            if (!AHEAD || __builtin_expect(hpos == HALO_FETCH, 0)) {
+                h = fetch<M, SH>(ap, i0 + ii - 2, j0 + jj - 2, k);
             } else {
-                int t2 = t - 4 * TY;
-                int side = t2 / (2 * TX), rem = t2 % (2 * TX);
-                int row = rem / TX, col = rem % TX;
-                jj = side ? TY + 2 + row : row;
-                ii = col + 2;
+                Prim P = decode_ideal<M>(hraw[0], hraw[1], hraw[2], hraw[3], hraw[4], IdealGas(ap->gas));
+                if (hpos < HALO_NONE) {
+                    if (SH && hS) P.a = -(P.a);
+                    if (hpos & HALO_FLIP0) P.v0 = -(P.v0);
+                    if (hpos & HALO_FLIP1) P.v1 = -(P.v1);
+                }
+                h = PrimT<R>{R(P.rho), R(P.v0), R(P.v1), R(P.v2), R(P.u), R(P.a)};
             }
-            PrimT<R> h = fetch<M, SH>(ap, i0 + ii - 2, j0 + jj - 2, k);
             const int s = jj * PX + ii;
             sP[0 * PLANE + s] = h.rho; sP[1 * PLANE + s] = h.v0; sP[2 * PLANE + s] = h.v1;
             sP[3 * PLANE + s] = h.v2; sP[4 * PLANE + s] = h.u; sP[5 * PLANE + s] = h.a;
@@ -666,26 +760,49 @@ __device__ __forceinline__ void stage_tile(int wg)
             side_flux<M, FLUX, JN, JT1, JT2>(LpJ, lds_side(sJ, NSJ, sj), gR, Fx, shock_opt<R>(ap));
             lds_put_flux(sJ, NSJ, sj, Fx);
         }
-        if (tidk < NBND) {
-            R Fx[5];
-            if (tidk < TY) {
-                if (j0 + tidk < ap->nj) {
-                    const int si = tidk * (TX + 1);
-                    side_flux<M, FLUX, 0, 1, 2>(lds_side(sLw, TY, tidk), lds_side(sI, NSI, si), gR, Fx,
-                                                shock_opt<R>(ap));
-                    lds_put_flux(sI, NSI, si, Fx);
-                }
-            } else {
-                const int c = tidk - TY;
-                if (i0 + c < ap->ni) {
-                    side_flux<M, FLUX, JN, JT1, JT2>(lds_side(sLs, TX, c), lds_side(sJ, NSJ, c), gR, Fx,
-                                                     shock_opt<R>(ap));
-                    lds_put_flux(sJ, NSJ, c, Fx);
-                }
+        // the tile's south faces are the first wave's, its west faces the
+        // second's (the last two had the halo cells' face states)
+        if (tidk < TX) {
+            const int c = tidk;
+            if (i0 + c < ap->ni) {
+                R Fx[5];
+                side_flux<M, FLUX, JN, JT1, JT2>(lds_side(sLs, TX, c), lds_side(sJ, NSJ, c), gR, Fx, shock_opt<R>(ap));
+                lds_put_flux(sJ, NSJ, c, Fx);
+            }
+        } else if (tidk >= 64 && tidk < 64 + TY) {
+            const int r = tidk - 64;
+            if (j0 + r < ap->nj) {
+                R Fx[5];
+                const int si = r * (TX + 1);
+                side_flux<M, FLUX, 0, 1, 2>(lds_side(sLw, TY, r), lds_side(sI, NSI, si), gR, Fx, shock_opt<R>(ap));
+                lds_put_flux(sI, NSI, si, Fx);
             }
         }
+        // the state of plane k + KRAW
+        auto k_state = [&](KArgs A) {
+            if (!raw_ok) return fetch<M, SH>(A, ik, jk, k + KRAW);
+            Prim P = decode_ideal<M>(raw[0], raw[1], raw[2], raw[3], raw[4], IdealGas(A->gas));
+            if (SH && A->S[cell_index(A, ik, jk, k + KRAW)]) P.a = -(P.a);
+            return PrimT<R>{R(P.rho), R(P.v0), R(P.v1), R(P.v2), R(P.u), R(P.a)};
+        };
+        // 4. k direction: face states of cell k+1 and the flux of the own cell's
+        // top face
+        if constexpr (DIMS == 3 && !KAHEAD) {
+            ap = args();
+            if (AHEAD && tidk < NHC && k + 1 < k1) halo_load(ap, k + 1);
+            const IdealGasT<R> gR = cast_gas<R>(IdealGas(ap->gas));
+            const PrimT<R> q2 = k_state(ap);
+            own = lds_prim(sP, PLANE, s0);
+            SideT<R> Lnext, Rnext;
+            recon_cell<M>(cast_wu<R>(L2R2U(ap->wu[2])), ho, lim, clip, own, qa, q2, Lnext, Rnext);
+            LpC.a = own.a;
+            if (own_k) side_flux<M, FLUX, 2, 0, 1>(LpC, Rnext, gR, Ft, shock_opt<R>(ap));
+            LpC = Lnext;
+            own = qa;
+            qa = q2;
+        }
         __syncthreads();
-        // 4. flux divergence in face order N, E, S, W, T, B (fvcell.d:789-825),
+        // 5. flux divergence in face order N, E, S, W, T, B (fvcell.d:789-825),
         // stage update, decode check, write; all in FP64.  Cells next to a
         // one-sided boundary are the boundary kernel's.
         ap = args();
@@ -730,20 +847,16 @@ __device__ __forceinline__ void stage_tile(int wg)
                 finish_cell<M>(ap, cell_index(ap, ik, jk, k), integ, ap->vol_inv, 0.0);
             }
         }
-        // 5. k-direction work for plane k+1: face states of cell k+2 and the
-        // flux of the top face of cell k+1
-        if constexpr (DIMS == 3) {
+        if constexpr (DIMS == 3 && !KAHEAD) {
+#pragma unroll
+            for (int q = 0; q < 5; ++q) Fb[q] = Ft[q];
+        }
+        // 6. KAHEAD: face states of cell k+2 and the flux of the top face of cell k+1
+        if constexpr (DIMS == 3 && KAHEAD) {
             if (k + 1 < k1) {
                 ap = args();
                 const IdealGasT<R> gR = cast_gas<R>(IdealGas(ap->gas));
-                PrimT<R> q3;
-                if (raw_ok) {
-                    Prim P = decode_ideal<M>(raw[0], raw[1], raw[2], raw[3], raw[4], IdealGas(ap->gas));
-                    if (SH && ap->S[cell_index(ap, ik, jk, k + 3)]) P.a = -(P.a);
-                    q3 = PrimT<R>{R(P.rho), R(P.v0), R(P.v1), R(P.v2), R(P.u), R(P.a)};
-                } else {
-                    q3 = fetch<M, SH>(ap, ik, jk, k + 3);
-                }
+                const PrimT<R> q3 = k_state(ap);
                 SideT<R> Lnext, Rnext;
                 recon_cell<M>(cast_wu<R>(L2R2U(ap->wu[2])), ho, lim, clip, qa, qb, q3, Lnext, Rnext);
 #pragma unroll
