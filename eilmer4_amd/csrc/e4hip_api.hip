@@ -302,6 +302,8 @@ std::vector<int> tune_key(const BlockH& b)
     return {b.ni, b.nj, b.nk, c.precision_mode, kernel_flux(c.flux_calculator), def};
 }
 
+bool mixed_fluxes() { return g_state.cfg.precision_mode == E4HIP_PRECISION_MIXED; }
+
 int kchunk_for(const BlockH& b)
 {
     const char* env = getenv("E4HIP_KCHUNK");
@@ -310,12 +312,10 @@ int kchunk_for(const BlockH& b)
     for (const auto& t : g_state.kchunk_tuned)
         if (t.first == key) return t.second;
     long nxy = (long)((b.ni + TILE_X - 1) / TILE_X) * ((b.nj + TILE_Y - 1) / TILE_Y);
-    // aim for >= 2048 workgroups (8 per CU) while marching at least 8 planes
+    // aim for >= 2048 workgroups (8 per CU)
     long chunks = (2048 + nxy - 1) / nxy;
-    long kc = (b.nk + chunks - 1) / chunks;
-    if (kc < 8) kc = 8;
-    if (kc > b.nk) kc = b.nk;
-    return (int)kc;
+    const int kc = (int)((b.nk + chunks - 1) / chunks);
+    return std::min(b.nk, mixed_fluxes() ? std::max(kc, 8) : kc);
 }
 
 int ensure_counters(int slots)
@@ -602,13 +602,45 @@ int launch_stage(const BlockH& b, int stage, double dt, unsigned int* counters)
 }
 
 // The k-chunk autotuner.  For a uniform 3D ideal-gas block whose shape has
-// not been tuned under the current arithmetic, the stage kernel of stage 1 is
-// timed (HIP events, three launches after a warm-up) at candidate chunk
-// heights -- the heights that split nk into 1, 2, 3, 4, 6, 8, 12, 16 or 32
-// chunks of at least four planes -- and the fastest is kept for that shape.
-// Stage 1 only reads U[0] and writes U[1], d[0] and counters that the step
-// resets, and every chunk height gives the same bits, so tuning before a step
-// changes its timing only.
+// not been tuned under the current arithmetic, the stages of the scheme are
+// timed (HIP events, after a warm-up) at candidate chunk heights and the fastest
+// is kept for that shape.  The stages only write U[1..], dUdt and counters that
+// the step resets, so tuning before a step changes its timing only -- except for the
+// last bits of the FP64 fast and mixed forms, whose loops and their peeled first
+// planes the compiler contracts differently.  In mixed precision that is an FP32
+// rounding of a flux, and the candidates stay the heights that split nk into 1, 2,
+// 3, 4, 6, 8, 12, 16 or 32 chunks of at least four planes.
+//
+// Chunks per block tried in FP64, and whether a launch of `wgs` workgroups is worth a
+// try where the block's heights give from `fewest` (whole columns) to `most`
+// (single planes): it fills the 256 compute units three deep, or as nearly as the
+// shape allows, and is not cut finer than 8192.  A short column costs two face
+// states and a flux per cell more than its share of a tall one, but small blocks
+// leave the chip idle otherwise: 61 x 45 x 37 hllc 46 us at four planes, 22 at
+// one; 128^3 adaptive_hanel_ausmdv 167 us at 11 planes (768 workgroups), 210 at
+// 16.
+constexpr int TUNE_CHUNKS[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 32, 48, 64, 96, 128, 256};
+constexpr int TUNE_CHUNKS_MIXED[] = {1, 2, 3, 4, 6, 8, 12, 16, 32};
+std::vector<int> tune_chunks()
+{
+    if (mixed_fluxes()) return {std::begin(TUNE_CHUNKS_MIXED), std::end(TUNE_CHUNKS_MIXED)};
+    return {std::begin(TUNE_CHUNKS), std::end(TUNE_CHUNKS)};
+}
+
+bool tune_worthwhile(long wgs, long fewest, long most)
+{
+    const long lo = std::min(768L, std::max(most / 2, 1L)), hi = std::max(8192L, fewest);
+    return wgs >= lo && wgs <= hi;
+}
+
+// Planes per workgroup of a block in a batched launch of `chunks` chunks a block.
+int batch_height(const BlockH& b, long chunks)
+{
+    if (b.dims != 3) return 1;
+    const int kc = (int)((b.nk + chunks - 1) / chunks);
+    return mixed_fluxes() ? std::min(std::max(kc, 4), b.nk) : kc;
+}
+
 std::vector<int> batch_tune_key(const std::vector<const BlockH*>& blks);
 int launch_stage_batch(const std::vector<const BlockH*>& blks, const std::vector<unsigned int*>& counters,
                        int stage, double dt, int set, long force_chunks);
@@ -629,10 +661,14 @@ int autotune_blocks(const int* blks, int nblk, double dt)
         bool known = false;
         for (const auto& t : g_state.kchunk_tuned) known = known || t.first == key;
         if (known) continue;
+        const long cols = (long)((b.ni + TILE_X - 1) / TILE_X) * ((b.nj + TILE_Y - 1) / TILE_Y);
         std::vector<int> cand;
-        for (int chunks : {1, 2, 3, 4, 6, 8, 12, 16, 32}) {
+        for (int chunks : tune_chunks()) {
             const int kc = (b.nk + chunks - 1) / chunks;
-            if (kc >= 4 && std::find(cand.begin(), cand.end(), kc) == cand.end()) cand.push_back(kc);
+            const bool worth = mixed_fluxes() ? kc >= 4
+                                              : tune_worthwhile(cols * ((b.nk + kc - 1) / kc), cols, cols * b.nk);
+            if (worth && std::find(cand.begin(), cand.end(), kc) == cand.end())
+                cand.push_back(kc);
         }
         if (cand.empty()) cand.push_back(b.nk);
         hipEvent_t e0, e1;
@@ -704,11 +740,26 @@ int autotune_blocks(const int* blks, int nblk, double dt)
                 HIP_TRY(hipEventCreate(&e1));
                 // as for one block: the scheme's stages in order, two rounds
                 const int ns = nstages(g_state.cfg.gasdynamic_update_scheme);
-                const long cand[] = {1L, 2L, 3L, 4L, 6L, 8L, 12L, 16L, 32L};
-                float cand_ms[sizeof(cand) / sizeof(cand[0])];
-                for (float& m : cand_ms) m = 1e30f;
+                long cols = 0, most = 0;
+                for (const BlockH* b : bl) {
+                    const long c = (long)((b->ni + TILE_X - 1) / TILE_X) * ((b->nj + TILE_Y - 1) / TILE_Y);
+                    cols += c;
+                    most += c * b->nk;
+                }
+                std::vector<long> cand;
+                for (int chunks : tune_chunks()) {
+                    long wgs = 0;
+                    for (const BlockH* b : bl) {
+                        const long kc = batch_height(*b, chunks);
+                        wgs += (long)((b->ni + TILE_X - 1) / TILE_X) * ((b->nj + TILE_Y - 1) / TILE_Y) *
+                               ((b->nk + kc - 1) / kc);
+                    }
+                    if (mixed_fluxes() || tune_worthwhile(wgs, cols, most)) cand.push_back(chunks);
+                }
+                if (cand.empty()) cand.push_back(1);
+                std::vector<float> cand_ms(cand.size(), 1e30f);
                 for (int round = 0; round < 2; ++round) {
-                    for (size_t ci = 0; ci < sizeof(cand) / sizeof(cand[0]); ++ci) {
+                    for (size_t ci = 0; ci < cand.size(); ++ci) {
                         auto pass = [&]() {
                             for (int st = 1; st <= ns; ++st) {
                                 int rc = launch_stage_batch(bl, cnt, st, dt, 0, cand[ci]);
@@ -731,9 +782,9 @@ int autotune_blocks(const int* blks, int nblk, double dt)
                         cand_ms[ci] = std::min(cand_ms[ci], ms);
                     }
                 }
-                long best = 1;
+                long best = cand[0];
                 float best_ms = 1e30f;
-                for (size_t ci = 0; ci < sizeof(cand) / sizeof(cand[0]); ++ci)
+                for (size_t ci = 0; ci < cand.size(); ++ci)
                     if (cand_ms[ci] < best_ms) { best_ms = cand_ms[ci]; best = cand[ci]; }
                 HIP_TRY(hipEventDestroy(e0));
                 HIP_TRY(hipEventDestroy(e1));
@@ -832,12 +883,7 @@ int launch_stage_batch(const std::vector<const BlockH*>& blks, const std::vector
     std::vector<long> ntile(n);
     for (int e = 0; e < n; ++e) {
         const BlockH& b = *blks[e];
-        int kc = 1;
-        if (b.dims == 3) {
-            kc = (int)((b.nk + chunks - 1) / chunks);
-            if (kc < 4) kc = 4;
-            if (kc > b.nk) kc = b.nk;
-        }
+        const int kc = batch_height(b, chunks);
         dim3 grid;
         int rc = stage_args_for(b, stage, dt, counters[e], kc, args[e], grid);
         if (rc) return rc;
