@@ -70,6 +70,17 @@ __device__ __forceinline__ long gen_face_index(const TPArgs& A, int d, int i, in
     return ((long)k * nfj + j) * nfi + i;
 }
 
+// The indices of element e of an array of n0 x n1 x (any) elements.  32-bit
+// divisions: a block's faces and cells number well below 2^29 (more than 400
+// bytes of device memory per cell).
+__device__ __forceinline__ void gen_indices(unsigned int e, int n0, int n1, int& i, int& j, int& k)
+{
+    const unsigned int row = e / (unsigned int)n0;
+    i = (int)(e - row * (unsigned int)n0);
+    k = (int)(row / (unsigned int)n1);
+    j = (int)(row - (unsigned int)k * (unsigned int)n1);
+}
+
 // Length in direction d of the stencil position (i, j, k), which may be a
 // ghost cell one or two layers outside the block: the ghost cells of a face
 // copy the lengths of the interior cells they mirror (sfluidblock.d:673-713),
@@ -105,6 +116,26 @@ __device__ __forceinline__ double gen_len(const TPArgs& A, int d, int i, int j, 
     return A.geo[(1 + d) * A.qs + ((long)sk * A.nj + sj) * A.ni + si];
 }
 
+// Length in direction DIR of the position p of a line (of n cells, cell 0 is c0,
+// step apart), in the block or a ghost whose length gen_len mirrors or wraps; with
+// `special` (a line with another kind of ghost) a ghost's is meaningless.
+template <int DIR>
+__device__ __forceinline__ double gen_line_len(const TPArgs& A, unsigned int c0, unsigned int step, int n, int p,
+                                               bool special)
+{
+    int src = p;
+    if (p < 0 || p >= n) {
+        const bool plus = p >= n;
+        const int layer = plus ? p - n + 1 : -p;
+        const int face = (DIR == 0) ? (plus ? FACE_EAST : FACE_WEST)
+                       : (DIR == 1) ? (plus ? FACE_NORTH : FACE_SOUTH) : (plus ? FACE_TOP : FACE_BOTTOM);
+        src = (plus != (A.bc->type[face] == BC_PERIODIC)) ? n - layer : layer - 1;
+        if (special) src = 0;
+    }
+    const unsigned int off = (c0 + (unsigned int)src * step) * 8u;
+    return *(const double*)((const char*)(A.geo + (long)(1 + DIR) * A.qs) + off);
+}
+
 // Global velocity of a stencil position reached along direction d from the
 // block; a slip-wall ghost (r.flip >= 0) is its mirrored cell's velocity
 // reflected about the boundary face at the ghost's in-face position.
@@ -125,11 +156,24 @@ __device__ __forceinline__ void gen_vel(const TPArgs& A, const TPRef& r, int d, 
     }
 }
 
-// l2r2_prepare (onedinterp.d:118-133) for one face
-template <class R>
+// l2r2_prepare (onedinterp.d:118-133) for one face; the plain FP64 form
+// multiplies by reciprocals good to an ulp.
+template <class M, class R>
 __device__ __forceinline__ L2R2WT<R> gen_l2r2_weights(double lenL1, double lenL0, double lenR0, double lenR1)
 {
     L2R2WT<R> w;
+    if constexpr (std::is_same<M, ModeFast64>::value) {
+        w.lenL0 = lenL0;
+        w.lenR0 = lenR0;
+        w.aL0 = 0.5 * lenL0 * rcp_full(lenL1 + 2.0 * lenL0 + lenR0);
+        w.aR0 = 0.5 * lenR0 * rcp_full(lenL0 + 2.0 * lenR0 + lenR1);
+        w.two_over_lenL0_plus_lenL1 = 2.0 * rcp_full(lenL0 + lenL1);
+        w.two_over_lenR0_plus_lenL0 = 2.0 * rcp_full(lenR0 + lenL0);
+        w.two_over_lenR1_plus_lenR0 = 2.0 * rcp_full(lenR1 + lenR0);
+        w.two_lenL0_plus_lenL1 = 2.0 * lenL0 + lenL1;
+        w.two_lenR0_plus_lenR1 = 2.0 * lenR0 + lenR1;
+        return w;
+    }
     w.lenL0 = R(lenL0);
     w.lenR0 = R(lenR0);
     w.aL0 = R(0.5 * lenL0 / (lenL1 + 2.0 * lenL0 + lenR0));
@@ -224,9 +268,9 @@ __device__ __forceinline__ void gen_flux(const TPArgs& A, const GSide<NSP>& L, c
     }
 }
 
-// One face of direction DIR per thread.
+// One face of direction DIR: f0, or none if it is beyond the last.
 template <class M, int NSP, int FLUX, int DIR>
-__global__ __launch_bounds__(128) void gen_face_kernel(TPArgs A)
+__device__ __forceinline__ void gen_face_body(const TPArgs& A, long f0)
 {
     using MR = typename std::conditional<NSP == 0, M, typename TPArith<M>::type>::type;
     using R = typename MR::R;
@@ -236,16 +280,15 @@ __global__ __launch_bounds__(128) void gen_face_kernel(TPArgs A)
     if (stage_aborted(A.abort_prev)) return;
     const int nfi = A.ni + (DIR == 0), nfj = A.nj + (DIR == 1), nfk = (A.dims == 3) ? A.nk + (DIR == 2) : 1;
     const long nf = (long)nfi * nfj * nfk;
-    const long f0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const bool active = f0 < nf;
     const long f = active ? f0 : nf - 1;   // idle lanes compute the last face and store nothing
-    const int i = (int)(f % nfi);
-    const int j = (int)((f / nfi) % nfj);
-    const int k = (int)(f / ((long)nfi * nfj));
+    int i, j, k;
+    gen_indices((unsigned int)f, nfi, nfj, i, j, k);
     const int di = (DIR == 0), dj = (DIR == 1), dk = (DIR == 2);
     const int pos = (DIR == 0) ? i : (DIR == 1) ? j : k;
     const int nD = (DIR == 0) ? A.ni : (DIR == 1) ? A.nj : A.nk;
     const GFrame fr = gen_frame(A, DIR, f);
+    auto ref = [&](int m) { return tp_ref(A, i + (m - 2) * di, j + (m - 2) * dj, k + (m - 2) * dk); };
     double F[NQ];
     int fe = 0, fb = 0;
     const int face_m = (DIR == 0) ? FACE_WEST : (DIR == 1) ? FACE_SOUTH : FACE_BOTTOM;
@@ -257,22 +300,69 @@ __global__ __launch_bounds__(128) void gen_face_kernel(TPArgs A)
         const TPRef rc = out_m ? tp_ref(A, i, j, k) : tp_ref(A, i - di, j - dj, k - dk);
         gen_outflow_flux<NSP>(rc, out_m ? -1 : 1, fr, F);
     } else {
-        TPRef r[4];
-        double v[4][3];
+        // The stencil's values, all loaded before any is used.  A position that
+        // is a cell of the block, or copies one, is a field's scalar base and a
+        // 32-bit offset; a lane with a position of another kind (inflow,
+        // connected, stored ghost) takes it from tp_ref afterwards, as it does a
+        // reflected velocity beyond a slip wall.  Resolving every position to a
+        // pointer first cost 5-8 % (150 x 80 x 72: 46.2, 41.5, 42.6 us for the
+        // i, j and k faces; 44.3, 38.4, 39.4 this way).
+        const TPStencil<DIR> st = tp_stencil<DIR>(A, i, j, k);
+        auto val = [&](int m, int field) {
+            return *(const double*)((const char*)(A.Pin + (long)field * A.qs) + st.off[m]);
+        };
+        const unsigned int step = (DIR == 0) ? 1u : (DIR == 1) ? (unsigned int)A.ni : (unsigned int)A.ni * A.nj;
+        const unsigned int c0 = (DIR == 0) ? ((unsigned int)k * A.nj + j) * A.ni
+                              : (DIR == 1) ? (unsigned int)k * A.nj * A.ni + i : (unsigned int)j * A.ni + i;
+        double v[4][3], rho[4], u[4], len[4], T[2], a[2];
+        double Y[4][NSP > 0 ? NSP : 1];
+        unsigned char sh[2] = {0, 0};
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
-            const int si = i + (m - 2) * di, sj = j + (m - 2) * dj, sk = k + (m - 2) * dk;
-            r[m] = tp_ref(A, si, sj, sk);
-            gen_vel(A, r[m], DIR, si, sj, sk, v[m]);
-            gen_to_local(v[m], fr);
+#pragma unroll
+            for (int d = 0; d < 3; ++d) v[m][d] = val(m, P_VX + d);
+            if (A.high_order) {
+                rho[m] = val(m, P_RHO);
+                u[m] = val(m, P_U);
+                len[m] = gen_line_len<DIR>(A, c0, step, nD, pos + m - 2, st.special);
+#pragma unroll
+                for (int q = 0; q < NSP; ++q) Y[m][q] = val(m, P_Y + q);
+            }
         }
+#pragma unroll
+        for (int sd = 0; sd < 2; ++sd) {
+            if (NSP > 0) T[sd] = val(1 + sd, P_T);
+            a[sd] = val(1 + sd, P_A);
+            if (FLUX == FLUX_SHOCK) {
+                const int p = pos + sd - 1;
+                sh[sd] = ((p < 0 || p >= nD) ? A.Sprev : A.S)[st.off[1 + sd] / 8u];
+            }
+        }
+        if (__builtin_expect(st.special || st.flip[0] || st.flip[1] || st.flip[2] || st.flip[3], 0)) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const int p = pos + m - 2;
+                if (p >= 0 && p < nD) continue;
+                const TPRef r = ref(m);
+                gen_vel(A, r, DIR, i + (m - 2) * di, j + (m - 2) * dj, k + (m - 2) * dk, v[m]);
+                rho[m] = tp_val(r, P_RHO);
+                u[m] = tp_val(r, P_U);
+                len[m] = gen_len(A, DIR, i + (m - 2) * di, j + (m - 2) * dj, k + (m - 2) * dk);
+#pragma unroll
+                for (int q = 0; q < NSP; ++q) Y[m][q] = tp_val(r, P_Y + q);
+                if (m == 1 || m == 2) {
+                    if (NSP > 0) T[m - 1] = tp_val(r, P_T);
+                    a[m - 1] = tp_val(r, P_A);
+                    if (FLUX == FLUX_SHOCK) sh[m - 1] = r.s ? *r.s : 0;
+                }
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < 4; ++m) gen_to_local(v[m], fr);
         GSide<NSP> Lf, Rf;
         bool okL = false, okR = false;
         if (A.high_order) {
-            double len[4];
-#pragma unroll
-            for (int m = 0; m < 4; ++m) len[m] = gen_len(A, DIR, i + (m - 2) * di, j + (m - 2) * dj, k + (m - 2) * dk);
-            const L2R2WT<R> w = gen_l2r2_weights<R>(len[0], len[1], len[2], len[3]);
+            const L2R2WT<R> w = gen_l2r2_weights<M, R>(len[0], len[1], len[2], len[3]);
             const bool lim = A.apply_limiter, clip = A.extrema_clipping;
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
@@ -284,24 +374,21 @@ __global__ __launch_bounds__(128) void gen_face_kernel(TPArgs A)
                 // (R is double for mixtures)
 #pragma unroll
                 for (int s = 0; s < NSP; ++s)
-                    interp_l2r2_scalar<MR>(w, lim, clip, tp_val(r[0], P_Y + s), tp_val(r[1], P_Y + s),
-                                           tp_val(r[2], P_Y + s), tp_val(r[3], P_Y + s), Lf.Y[s], Rf.Y[s]);
+                    interp_l2r2_scalar<MR>(w, lim, clip, Y[0][s], Y[1][s], Y[2][s], Y[3][s], Lf.Y[s], Rf.Y[s]);
                 if (scale_mass_fractions<MR, NSP>(Lf.Y) != 0) {
 #pragma unroll
-                    for (int s = 0; s < NSP; ++s) Lf.Y[s] = tp_val(r[1], P_Y + s);
+                    for (int s = 0; s < NSP; ++s) Lf.Y[s] = Y[1][s];
                 }
                 if (scale_mass_fractions<MR, NSP>(Rf.Y) != 0) {
 #pragma unroll
-                    for (int s = 0; s < NSP; ++s) Rf.Y[s] = tp_val(r[2], P_Y + s);
+                    for (int s = 0; s < NSP; ++s) Rf.Y[s] = Y[2][s];
                 }
             }
             {
                 R qL, qR;
-                interp_l2r2_scalar<MR>(w, lim, clip, R(tp_val(r[0], P_RHO)), R(tp_val(r[1], P_RHO)),
-                                       R(tp_val(r[2], P_RHO)), R(tp_val(r[3], P_RHO)), qL, qR);
+                interp_l2r2_scalar<MR>(w, lim, clip, R(rho[0]), R(rho[1]), R(rho[2]), R(rho[3]), qL, qR);
                 Lf.rho = qL; Rf.rho = qR;
-                interp_l2r2_scalar<MR>(w, lim, clip, R(tp_val(r[0], P_U)), R(tp_val(r[1], P_U)), R(tp_val(r[2], P_U)),
-                                       R(tp_val(r[3], P_U)), qL, qR);
+                interp_l2r2_scalar<MR>(w, lim, clip, R(u[0]), R(u[1]), R(u[2]), R(u[3]), qL, qR);
                 Lf.u = qL; Rf.u = qR;
             }
             // update_thermo_from_rhou on each side; on failure the side is its
@@ -309,31 +396,30 @@ __global__ __launch_bounds__(128) void gen_face_kernel(TPArgs A)
             // cell's (sfluidblock.d:2199-2208)
             if constexpr (NSP == 0) {
                 if (Lf.u > 0.0 && Lf.rho > 0.0) {
-                    Lf.T = Lf.u * A.ig.Cvinv; Lf.p = Lf.rho * A.ig.Rgas * Lf.T; Lf.a = tp_val(r[1], P_A); okL = true;
+                    Lf.T = Lf.u * A.ig.Cvinv; Lf.p = Lf.rho * A.ig.Rgas * Lf.T; Lf.a = a[0]; okL = true;
                 }
                 if (Rf.u > 0.0 && Rf.rho > 0.0) {
-                    Rf.T = Rf.u * A.ig.Cvinv; Rf.p = Rf.rho * A.ig.Rgas * Rf.T; Rf.a = tp_val(r[2], P_A); okR = true;
+                    Rf.T = Rf.u * A.ig.Cvinv; Rf.p = Rf.rho * A.ig.Rgas * Rf.T; Rf.a = a[1]; okR = true;
                 }
             } else {
                 using MA = typename TPArith<M>::type;
 #pragma nounroll
                 for (int sd = 0; sd < 2; ++sd) {
-                    const TPRef rc = sd ? r[2] : r[1];
                     TPState<NSP> Q;
                     Q.rho = sd ? Rf.rho : Lf.rho;
                     Q.u = sd ? Rf.u : Lf.u;
-                    Q.T = tp_val(rc, P_T);
+                    Q.T = T[sd];
 #pragma unroll
                     for (int s = 0; s < NSP; ++s) Q.Y[s] = sd ? Rf.Y[s] : Lf.Y[s];
                     if (tp_face_eos<MA, NSP, kPolish>(tp_gas(A), Q, &fe, &fb) == 0) {
-                        const double a = tp_val(rc, P_A);
-                        if (sd == 0) { Lf.T = Q.T; Lf.u = Q.u; Lf.p = Q.p; Lf.a = a; okL = true; }
-                        else { Rf.T = Q.T; Rf.u = Q.u; Rf.p = Q.p; Rf.a = a; okR = true; }
+                        const double as = a[sd];
+                        if (sd == 0) { Lf.T = Q.T; Lf.u = Q.u; Lf.p = Q.p; Lf.a = as; okL = true; }
+                        else { Rf.T = Q.T; Rf.u = Q.u; Rf.p = Q.p; Rf.a = as; okR = true; }
                     }
                 }
             }
-            if (!okL) gen_cell_side<NSP>(r[1], v[1], Lf);
-            if (!okR) gen_cell_side<NSP>(r[2], v[2], Rf);
+            if (!okL) gen_cell_side<NSP>(ref(1), v[1], Lf);
+            if (!okR) gen_cell_side<NSP>(ref(2), v[2], Rf);
             if constexpr (kExact) {
                 // the reconstruction hands its states over in the global frame
                 // and the flux calculator turns them back into the face frame
@@ -341,10 +427,10 @@ __global__ __launch_bounds__(128) void gen_face_kernel(TPArgs A)
                 gen_to_local(Lf.v, fr); gen_to_local(Rf.v, fr);
             }
         } else {
-            gen_cell_side<NSP>(r[1], v[1], Lf);
-            gen_cell_side<NSP>(r[2], v[2], Rf);
+            gen_cell_side<NSP>(ref(1), v[1], Lf);
+            gen_cell_side<NSP>(ref(2), v[2], Rf);
         }
-        const bool shock = (FLUX == FLUX_SHOCK) && ((r[1].s && *r[1].s) || (r[2].s && *r[2].s));
+        const bool shock = (FLUX == FLUX_SHOCK) && (sh[0] || sh[1]);
         gen_flux<M, NSP, FLUX>(A, Lf, Rf, shock, F);
         double m[3] = {F[1], F[2], F[3]};
         gen_to_global(m, fr);
@@ -368,6 +454,53 @@ __global__ __launch_bounds__(128) void gen_face_kernel(TPArgs A)
         if (__lane_id() == 0) {
             add_stat(A.stats, STAT_FACE_EVALS, (unsigned int)fe);
             add_stat(A.stats, STAT_FACE_FALLBACKS, (unsigned int)fb);
+        }
+    }
+}
+
+// One face of direction DIR per thread.
+template <class M, int NSP, int FLUX, int DIR>
+__global__ __launch_bounds__(128) void gen_face_kernel(TPArgs A)
+{
+    gen_face_body<M, NSP, FLUX, DIR>(A, (long)xcd_contiguous((int)blockIdx.x, (int)gridDim.x) * 128 + threadIdx.x);
+}
+
+// The faces of all directions in one launch (ideal gas).  Bound by memory: 168
+// bytes a face without reuse.  Consecutive workgroups of an XCD take the i, j and k
+// faces of about the same cells, whose states then come from its L2, and there is
+// one launch's last wave instead of three: 150 x 80 x 72 adaptive_hanel_ausmdv
+// 106 us against 44 + 38 + 39 in three launches, each XCD with a contiguous run of
+// faces, and 46 + 50 + 48 with the faces dealt to the XCDs in turn.  The update and
+// the detector read their j and k neighbours' faces and cells: contiguous runs took
+// them from 65 to 60 and from 46 to 36 us.  (Mixtures keep a launch a direction:
+// the temperature solves, not memory, set their time.)
+template <class M, int FLUX>
+__global__ __launch_bounds__(128) void gen_faces_kernel(TPArgs args)
+{
+    // (read through the kernarg segment: three bodies that index its arrays had
+    // the compiler copy the argument to scratch)
+#if defined(__HIP_DEVICE_COMPILE__)
+    const TPArgs& A = *(const TPArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+#else
+    const TPArgs& A = args;
+#endif
+    const int w = xcd_contiguous((int)blockIdx.x, (int)gridDim.x);
+    if (A.dims == 3) {
+        const long f0 = (long)(w / 3) * 128;
+        const int d = w % 3;
+        if (d == 0) {
+            if (f0 < (long)(A.ni + 1) * A.nj * A.nk) gen_face_body<M, 0, FLUX, 0>(A, f0 + threadIdx.x);
+        } else if (d == 1) {
+            if (f0 < (long)A.ni * (A.nj + 1) * A.nk) gen_face_body<M, 0, FLUX, 1>(A, f0 + threadIdx.x);
+        } else {
+            if (f0 < (long)A.ni * A.nj * (A.nk + 1)) gen_face_body<M, 0, FLUX, 2>(A, f0 + threadIdx.x);
+        }
+    } else {
+        const long f0 = (long)(w / 2) * 128;
+        if (w % 2 == 0) {
+            if (f0 < (long)(A.ni + 1) * A.nj) gen_face_body<M, 0, FLUX, 0>(A, f0 + threadIdx.x);
+        } else {
+            if (f0 < (long)A.ni * (A.nj + 1)) gen_face_body<M, 0, FLUX, 1>(A, f0 + threadIdx.x);
         }
     }
 }
@@ -460,12 +593,13 @@ __global__ __launch_bounds__(128) void ig_update_kernel(TPArgs A)
 {
     if (stage_aborted(A.abort_prev)) return;
     const long ncells = (long)A.ni * A.nj * A.nk;
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long c = (long)xcd_contiguous((int)blockIdx.x, (int)gridDim.x) * blockDim.x + threadIdx.x;
     const bool active = c < ncells;
     bool invalid = false, decode_fail = false;
     if (active) {
         const long qs = A.qs;
-        const int i = (int)(c % A.ni), j = (int)((c / A.ni) % A.nj), k = (int)(c / ((long)A.ni * A.nj));
+        int i, j, k;
+        gen_indices((unsigned int)c, A.ni, A.nj, i, j, k);
         double integ[5];
         gen_integral<5>(A, c, i, j, k, integ);
         const double vol_inv = 1.0 / A.geo[c];
@@ -538,9 +672,10 @@ __global__ __launch_bounds__(128) void gen_shock_detect_kernel(TPArgs A)
     using MD = typename std::conditional<M::kFast, ModeFast64, ModeExact>::type;
     if (stage_aborted(A.abort_prev)) return;
     const long n = (long)A.ni * A.nj * A.nk;
-    const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long c = (long)xcd_contiguous((int)blockIdx.x, (int)gridDim.x) * blockDim.x + threadIdx.x;
     if (c >= n) return;
-    const int i = (int)(c % A.ni), j = (int)((c / A.ni) % A.nj), k = (int)(c / ((long)A.ni * A.nj));
+    int i, j, k;
+    gen_indices((unsigned int)c, A.ni, A.nj, i, j, k);
     const TPRef own = tp_ref(A, i, j, k);
     const double tol = A.compression_tol;
     bool S = false;
@@ -582,7 +717,8 @@ static __global__ __launch_bounds__(256) void gen_cfl_kernel(TPArgs A, int strin
     const long qs = A.qs;
     double sig = 0.0;
     for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < ncells; c += (long)gridDim.x * blockDim.x) {
-        const int i = (int)(c % A.ni), j = (int)((c / A.ni) % A.nj), k = (int)(c / ((long)A.ni * A.nj));
+        int i, j, k;
+        gen_indices((unsigned int)c, A.ni, A.nj, i, j, k);
         const double* P = A.Pin;
         const double v[3] = {P[P_VX * qs + c], P[P_VY * qs + c], P[P_VZ * qs + c]};
         const double a = P[P_A * qs + c];
@@ -633,6 +769,12 @@ void launch_gen_faces(const TPArgs& A, hipStream_t stream)
     const long nf2 = (long)A.ni * A.nj * (A.nk + 1);
     const dim3 b(128);
     auto g = [](long n) { return dim3((unsigned)((n + 127) / 128)); };
+    if constexpr (NSP == 0) {
+        const int nd = (A.dims == 3) ? 3 : 2;
+        const long most = std::max(std::max(nf0, nf1), (nd == 3) ? nf2 : 0L);
+        hipLaunchKernelGGL((gen_faces_kernel<M, FLUX>), dim3(g(most).x * nd), b, 0, stream, A);
+        return;
+    }
     hipLaunchKernelGGL((gen_face_kernel<M, NSP, FLUX, 0>), g(nf0), b, 0, stream, A);
     hipLaunchKernelGGL((gen_face_kernel<M, NSP, FLUX, 1>), g(nf1), b, 0, stream, A);
     if (A.dims == 3) hipLaunchKernelGGL((gen_face_kernel<M, NSP, FLUX, 2>), g(nf2), b, 0, stream, A);
