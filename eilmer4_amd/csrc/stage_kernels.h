@@ -30,7 +30,7 @@
 //      state happen in registers.
 //
 // The FP64 form is bound by FP64 issue: a cell takes about 1100 vector
-// instructions and the kernel keeps the units three quarters busy at the 12 waves a
+// instructions and the kernel keeps the units 70 % busy at the 12 waves a
 // compute unit that 168 registers and 48 KB of LDS allow; a spill or a lower
 // occupancy costs more than the operations it saves.  256^3 ausmdv, one stage:
 // 1.252 ms; 1.065 with the shorter reconstruction and flux; 1.015 with the
