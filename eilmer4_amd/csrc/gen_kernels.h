@@ -768,16 +768,16 @@ void launch_gen_faces(const TPArgs& A, hipStream_t stream)
     const long nf0 = (long)(A.ni + 1) * A.nj * nfk, nf1 = (long)A.ni * (A.nj + 1) * nfk;
     const long nf2 = (long)A.ni * A.nj * (A.nk + 1);
     const dim3 b(128);
-    auto g = [](long n) { return dim3((unsigned)((n + 127) / 128)); };
+    auto g = [](long n) { return (unsigned)((n + 127) / 128); };
     if constexpr (NSP == 0) {
         const int nd = (A.dims == 3) ? 3 : 2;
         const long most = std::max(std::max(nf0, nf1), (nd == 3) ? nf2 : 0L);
-        hipLaunchKernelGGL((gen_faces_kernel<M, FLUX>), dim3(g(most).x * nd), b, 0, stream, A);
-        return;
+        hipLaunchKernelGGL((gen_faces_kernel<M, FLUX>), dim3(g(most) * nd), b, 0, stream, A);
+    } else {
+        hipLaunchKernelGGL((gen_face_kernel<M, NSP, FLUX, 0>), dim3(g(nf0)), b, 0, stream, A);
+        hipLaunchKernelGGL((gen_face_kernel<M, NSP, FLUX, 1>), dim3(g(nf1)), b, 0, stream, A);
+        if (A.dims == 3) hipLaunchKernelGGL((gen_face_kernel<M, NSP, FLUX, 2>), dim3(g(nf2)), b, 0, stream, A);
     }
-    hipLaunchKernelGGL((gen_face_kernel<M, NSP, FLUX, 0>), g(nf0), b, 0, stream, A);
-    hipLaunchKernelGGL((gen_face_kernel<M, NSP, FLUX, 1>), g(nf1), b, 0, stream, A);
-    if (A.dims == 3) hipLaunchKernelGGL((gen_face_kernel<M, NSP, FLUX, 2>), g(nf2), b, 0, stream, A);
 }
 
 template <class M, int NSP>
