@@ -4,6 +4,7 @@
 #include "gasdyn_device.h"
 #include "tp_gas_device.h"
 #include "learned_eos.h"
+#include "block_index.h"
 
 namespace e4 {
 

@@ -1436,10 +1436,12 @@ __global__ __launch_bounds__(64 * SD_TY) void shock_detect_kernel(
     if (jp >= nj) jp = sd_source(A->bc->type[FACE_NORTH], true, nj, &pflip, &pspecial);
     const long qs = A->qs;
     const double* __restrict__ U = A->Us;
+    // row (jj, kk) at the lane's column (a cell's byte offset passes 32 bits from 2^29
+    // cells on, which is 87 GB under pc)
     auto load = [&](int jj, int kk, double r[5]) {
-        const unsigned int off = (((unsigned int)kk * nj + jj) * ni + ic) * 8u;
+        const double* p = U + ic + row_start(ni, nj, jj, kk);
 #pragma unroll
-        for (int q = 0; q < 5; ++q) r[q] = *(const double*)((const char*)(U + q * qs) + off);
+        for (int q = 0; q < 5; ++q) r[q] = p[q * qs];
     };
     // plane kk of the lane's column, with what its k ghosts copy
     auto load_column = [&](int kk, double r[5], bool* flip, bool* special) {
