@@ -21,4 +21,19 @@ E4_HD long row_start(int ni, int nj, int j, int k)
     return (long)((unsigned long)((unsigned int)k * (unsigned int)nj + (unsigned int)j) * (unsigned int)ni);
 }
 
+// A load from a scalar 64-bit base with an unsigned 32-bit byte offset takes no vector
+// address arithmetic, and reaches 2^29 doubles.  Whether that is every cell of a block
+// and every face of each of its directions (a field of one double per cell or face):
+// blocks with a flow-state array and face fluxes take 482 bytes a cell and more, 259 GB
+// at 2^29 cells, so larger ones can fit the memory, and kernels that use such offsets
+// have another route for them.
+constexpr long OFFSET32_DOUBLES = 1L << 29;
+E4_HD bool offsets_reach_block(int dims, int ni, int nj, int nk)
+{
+    const long k = (dims == 3) ? nk : 1;
+    const long fi = (ni + 1L) * nj * k, fj = ni * (nj + 1L) * k, fk = (dims == 3) ? (long)ni * nj * (k + 1) : 0;
+    const long most = (fi > fj) ? ((fi > fk) ? fi : fk) : ((fj > fk) ? fj : fk);
+    return most <= OFFSET32_DOUBLES;
+}
+
 } // namespace e4

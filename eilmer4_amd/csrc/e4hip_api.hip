@@ -47,6 +47,7 @@ struct BlockH {
     long ncells = 0, qs = 0;
     int nq = 5;
     int nsp = 1;
+    bool wide = false;                            // 32-bit byte offsets do not reach every cell and face
     // U[0] is the current state; stage s writes U[s], and a step that ends
     // without bad cells swaps U[0] and U[stages] (simcore.d:2936-2941), so a
     // step that stops leaves U[0] as it was
@@ -995,6 +996,7 @@ int tp_args_for(const BlockH& b, int stage, double dt, unsigned int* counters, e
     A.qs = b.qs;
     for (int dd = 0; dd < 3; ++dd) { A.F[dd] = b.F[dd]; A.fqs[dd] = b.fqs[dd]; }
     A.ni = b.ni; A.nj = b.nj; A.nk = (b.dims == 3) ? b.nk : 1; A.dims = b.dims;
+    A.wide = b.wide;
     A.stage = stage;
     A.high_order = cfg.interpolation_order > 1;
     A.apply_limiter = cfg.apply_limiter;
@@ -1547,6 +1549,8 @@ int create_block(int gm, int dims, int ni, int nj, int nk, double dx, double dy,
     b.nsp = g_state.gases[gm].nsp;
     b.nq = (b.nsp > 1) ? 5 + b.nsp : 5;
     b.general = geom != nullptr;
+    const char* wide = getenv("E4HIP_WIDE_OFFSETS");   // gives any block the route of the largest
+    b.wide = !e4::offsets_reach_block(dims, ni, nj, nk) || (wide && atoi(wide) > 0);
     if (b.general) {
         // every cell needs a positive volume and positive lengths
         const long nc = b.ncells;

@@ -71,8 +71,8 @@ __device__ __forceinline__ long gen_face_index(const TPArgs& A, int d, int i, in
 }
 
 // The indices of element e of an array of n0 x n1 x (any) elements.  32-bit
-// divisions: a block's faces and cells number well below 2^29 (more than 400
-// bytes of device memory per cell).
+// divisions: a block's faces and cells number below 2^32 (480 bytes of device memory
+// per cell or more).
 __device__ __forceinline__ void gen_indices(unsigned int e, int n0, int n1, int& i, int& j, int& k)
 {
     const unsigned int row = e / (unsigned int)n0;
@@ -304,7 +304,8 @@ __device__ __forceinline__ void gen_face_body(const TPArgs& A, long f0)
         // is a cell of the block, or copies one, is a field's scalar base and a
         // 32-bit offset; a lane with a position of another kind (inflow,
         // connected, stored ghost) takes it from tp_ref afterwards, as it does a
-        // reflected velocity beyond a slip wall.  Resolving every position to a
+        // reflected velocity beyond a slip wall, and as every position is taken in a
+        // block that the offsets do not reach.  Resolving every position to a
         // pointer first cost 5-8 % (150 x 80 x 72: 46.2, 41.5, 42.6 us for the
         // i, j and k faces; 44.3, 38.4, 39.4 this way).
         const TPStencil<DIR> st = tp_stencil<DIR>(A, i, j, k);
@@ -342,7 +343,7 @@ __device__ __forceinline__ void gen_face_body(const TPArgs& A, long f0)
 #pragma unroll
             for (int m = 0; m < 4; ++m) {
                 const int p = pos + m - 2;
-                if (p >= 0 && p < nD) continue;
+                if (p >= 0 && p < nD && !A.wide) continue;
                 const TPRef r = ref(m);
                 gen_vel(A, r, DIR, i + (m - 2) * di, j + (m - 2) * dj, k + (m - 2) * dk, v[m]);
                 rho[m] = tp_val(r, P_RHO);

@@ -251,6 +251,7 @@ struct TPArgs {
     long qs;
     long fqs[3];
     int ni, nj, nk, dims;
+    int wide;                         // 32-bit byte offsets do not reach the block (offsets_reach_block)
     int stage;
     int high_order, apply_limiter, extrema_clipping;
     double c1, dt, g1, g2, g3;

@@ -193,9 +193,10 @@ __device__ __forceinline__ TPRef tp_ref(const TPArgs& A, int i, int j, int k)
 
 // The four stencil positions of a face of direction DIR as cells of the block:
 // byte offsets of the cells within a field, whether a position mirrors a slip
-// wall's cell (its normal velocity is negated), and whether the face reads a
-// state that is not a cell of the block (an inflow, a connected block's cell, a
-// stored ghost cell), for which the offsets mean nothing.  The same mapping as
+// wall's cell (its normal velocity is negated), and whether some position's offset
+// means nothing: the face reads a state that is not a cell of the block (an inflow,
+// a connected block's cell, a stored ghost cell), or the block has more cells than
+// the offsets reach (they then lead to another of its cells).  The same mapping as
 // tp_ref.
 template <int DIR>
 struct TPStencil {
@@ -214,7 +215,7 @@ __device__ __forceinline__ TPStencil<DIR> tp_stencil(const TPArgs& A, int i, int
     // cell 0 of the face's line along DIR
     const unsigned int c0 = (DIR == 0) ? ((unsigned int)k * A.nj + j) * A.ni
                           : (DIR == 1) ? (unsigned int)k * A.nj * A.ni + i : (unsigned int)j * A.ni + i;
-    st.special = false;
+    st.special = A.wide != 0;
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
         const int p = pos + m - 2;
@@ -661,8 +662,7 @@ __device__ __forceinline__ void tp_face_body(const TPArgs& A, long f0)
     using R = typename MF::R;
     constexpr bool kPolish = TPArith<M>::polish;
     if (stage_aborted(A.abort_prev)) return;
-    // (a block's faces and cells number well below 2^29, so that 32-bit byte
-    // offsets reach them: 768 bytes of device memory per cell)
+    // (cells and faces number below 2^32: 480 bytes of device memory per cell or more)
     const int nfi = A.ni + (DIR == 0), nfj = A.nj + (DIR == 1), nfk = (A.dims == 3) ? A.nk + (DIR == 2) : 1;
     const unsigned int nf = (unsigned int)nfi * nfj * nfk;
     const bool active = f0 < (long)nf;
@@ -821,7 +821,11 @@ __device__ __forceinline__ void tp_face_body(const TPArgs& A, long f0)
             FS* dst = reinterpret_cast<FS*>(A.F[DIR]);
             const long fq = A.fqs[DIR];
             const unsigned int off = f * (unsigned int)sizeof(FS);
-            auto put = [&](int q, FS x) { *(FS*)((char*)(dst + (long)q * fq) + off) = x; };
+            auto put = [&](int q, FS x) {
+                FS* const base = dst + (long)q * fq;
+                if (__builtin_expect(A.wide, 0)) base[f] = x;
+                else *(FS*)((char*)base + off) = x;
+            };
             put(0, F[0]);
             put(1 + pn, F[1]);
             put(1 + pt1, F[2]);

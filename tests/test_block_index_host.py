@@ -12,6 +12,7 @@ CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
 SOURCE = """
 #include "block_index.h"
 extern "C" {
+int reach_block(int d, int ni, int nj, int nk) { return e4::offsets_reach_block(d, ni, nj, nk); }
 long row_start(int ni, int nj, int j, int k) { return e4::row_start(ni, nj, j, k); }
 }
 """
@@ -35,3 +36,15 @@ def test_rows(lib, n):
     rng = random.Random(ni)
     for j, k in [(0, 0), (nj - 1, 0), (0, nk - 1), (nj - 1, nk - 1)] + [(rng.randrange(nj), rng.randrange(nk)) for _ in range(50)]:
         assert lib.row_start(ni, nj, j, k) == (k * nj + j) * ni
+
+
+@pytest.mark.parametrize("n", [(812, 812, 813), (813, 813, 813), (820, 820, 820), (23170, 23170, 1), (23171, 23170, 1),
+                               (2 ** 28 - 1, 2, 1), (2 ** 28, 2, 1), (2, 2 ** 28, 1), (2, 2, 2 ** 27), (2, 2, 2 ** 27 - 1),
+                               (2 ** 31 - 1, 2, 1), (128, 128, 128)])
+def test_blocks_out_of_reach(lib, n):
+    """The byte offset of every cell and face within its field is below 2^32 exactly where
+    the rule says so."""
+    ni, nj, nk = n
+    dims = 2 if nk == 1 else 3
+    most = max((ni + 1) * nj * nk, ni * (nj + 1) * nk, ni * nj * (nk + 1) if dims == 3 else 0)
+    assert bool(lib.reach_block(dims, ni, nj, nk)) == (8 * (most - 1) < 2 ** 32)
