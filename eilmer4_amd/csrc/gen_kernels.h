@@ -409,11 +409,11 @@ __device__ __forceinline__ void gen_face_body(const TPArgs& A, long f0)
                     TPState<NSP> Q;
                     Q.rho = sd ? Rf.rho : Lf.rho;
                     Q.u = sd ? Rf.u : Lf.u;
-                    Q.T = T[sd];
+                    Q.T = sd ? T[1] : T[0];   // (indexed by sd, T and a would live in scratch)
 #pragma unroll
                     for (int s = 0; s < NSP; ++s) Q.Y[s] = sd ? Rf.Y[s] : Lf.Y[s];
                     if (tp_face_eos<MA, NSP, kPolish>(tp_gas(A), Q, &fe, &fb) == 0) {
-                        const double as = a[sd];
+                        const double as = sd ? a[1] : a[0];
                         if (sd == 0) { Lf.T = Q.T; Lf.u = Q.u; Lf.p = Q.p; Lf.a = as; okL = true; }
                         else { Rf.T = Q.T; Rf.u = Q.u; Rf.p = Q.p; Rf.a = as; okR = true; }
                     }
