@@ -459,11 +459,15 @@ __device__ __forceinline__ void gen_face_body(const TPArgs& A, long f0)
     }
 }
 
-// One face of direction DIR per thread.
+// One face of direction DIR per thread (mixtures).  The workgroups are dealt to the
+// XCDs in turn: the temperature solves set the time, and a contiguous run of faces,
+// whose solves differ from another's in cost, leaves some XCDs waiting.  96 x 80 x 72
+// five-species ausmdv, a step: 784 us this way, 881 with contiguous runs; mixed 636,
+// 709; fp64_exact 6409, 7214.  (2D 600 x 400: 252, 244; 1500 x 1000: 1042, 1077.)
 template <class M, int NSP, int FLUX, int DIR>
 __global__ __launch_bounds__(128) void gen_face_kernel(TPArgs A)
 {
-    gen_face_body<M, NSP, FLUX, DIR>(A, (long)xcd_contiguous((int)blockIdx.x, (int)gridDim.x) * 128 + threadIdx.x);
+    gen_face_body<M, NSP, FLUX, DIR>(A, (long)blockIdx.x * 128 + threadIdx.x);
 }
 
 // The faces of all directions in one launch (ideal gas).  Bound by memory: 168
