@@ -5,6 +5,8 @@ Translation units, compiled in parallel:
                     reference's roundings (bit-identical to the CPU oracle)
   tp_exact.hip      -ffp-contract=off: the same for the thermally perfect mixture
   stage_fast64.hip  -ffp-contract=fast: the plain FP64 ideal-gas kernels
+  stage_fast64_3d.hip  -ffp-contract=on: the 3D stage kernels among them, whose
+                    results may not depend on how their planes are divided
   stage_mixed.hip   -ffp-contract=fast: the mixed FP32/FP64 ideal-gas kernels
   tp_fast.hip       -ffp-contract=fast: the plain and mixed mixture kernels and
                     the learned-guess inference
@@ -31,6 +33,7 @@ COMMON = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Xclang", "-ta
 UNITS = [("stage_exact.hip", ["-ffp-contract=off"]),
          ("tp_exact.hip", ["-ffp-contract=off"]),
          ("stage_fast64.hip", ["-ffp-contract=fast"]),
+         ("stage_fast64_3d.hip", ["-ffp-contract=on"]),
          ("stage_mixed.hip", ["-ffp-contract=fast"]),
          ("tp_fast.hip", ["-ffp-contract=fast"]),
          ("gen_exact.hip", ["-ffp-contract=off"]),

@@ -606,11 +606,13 @@ int launch_stage(const BlockH& b, int stage, double dt, unsigned int* counters)
 // not been tuned under the current arithmetic, the stages of the scheme are
 // timed (HIP events, after a warm-up) at candidate chunk heights and the fastest
 // is kept for that shape.  The stages only write U[1..], dUdt and counters that
-// the step resets, so tuning before a step changes its timing only -- except for the
-// last bits of the FP64 fast and mixed forms, whose loops and their peeled first
-// planes the compiler contracts differently.  In mixed precision that is an FP32
-// rounding of a flux, and the candidates stay the heights that split nk into 1, 2,
-// 3, 4, 6, 8, 12, 16 or 32 chunks of at least four planes.
+// the step resets, and no height changes a bit of the FP64 forms' results (the
+// exact form does not contract, the plain form contracts alike in every copy of an
+// expression: stage_fast64_3d.hip), so tuning before a step changes its timing
+// only.  The mixed form's loop and its peeled first planes are contracted
+// differently: there the height moves an FP32 rounding of a flux, and the candidates
+// stay the heights that split nk into 1, 2, 3, 4, 6, 8, 12, 16 or 32 chunks of at
+// least four planes.
 //
 // Chunks per block tried in FP64, and whether a launch of `wgs` workgroups is worth a
 // try where the block's heights give from `fewest` (whole columns) to `most`

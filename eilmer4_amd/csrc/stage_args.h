@@ -309,9 +309,11 @@ struct TPArgs {
 };
 
 // Launchers, one per arithmetic mode; each lives in its own translation unit
-// (stage_exact.hip is compiled without FMA contraction, stage_fast.hip with it).
+// (the exact ones are compiled without FMA contraction, the others with it; the 3D
+// stage kernels of the plain FP64 form in one of their own, see there).
 void launch_stage_exact(const StageArgs& A, dim3 grid, hipStream_t stream, int dims, int flux);
 void launch_stage_fast64(const StageArgs& A, dim3 grid, hipStream_t stream, int dims, int flux);
+void launch_stage_fast64_3d(const StageArgs& A, dim3 grid, hipStream_t stream, int flux);
 void launch_stage_mixed(const StageArgs& A, dim3 grid, hipStream_t stream, int dims, int flux);
 // batched: nwg workgroups over the blocks of one table (same dims; default
 // reconstruction options or not, for all of them)
@@ -324,6 +326,7 @@ void launch_boundary_cells_batch_exact(const BatchArgs& B, int nwg, hipStream_t 
 void launch_boundary_cells_batch_fast64(const BatchArgs& B, int nwg, hipStream_t stream, int dims, int flux);
 void launch_boundary_cells_batch_mixed(const BatchArgs& B, int nwg, hipStream_t stream, int dims, int flux);
 void launch_stage_batch_fast64(const BatchArgs& B, int nwg, bool def, hipStream_t stream, int dims, int flux);
+void launch_stage_batch_fast64_3d(const BatchArgs& B, int nwg, bool def, hipStream_t stream, int flux);
 void launch_stage_batch_mixed(const BatchArgs& B, int nwg, bool def, hipStream_t stream, int dims, int flux);
 // thermally perfect mixture (five species): faces of every direction, then the
 // update; decode of an uploaded state

@@ -1,4 +1,5 @@
-// stage_fast64.hip -- stage-kernel instantiations for ModeFast64 (the plain FP64 form).
+// stage_fast64.hip -- instantiations for ModeFast64 (the plain FP64 form): the 2D stage
+// kernels, boundary cells and shock detector (the 3D stage kernels: stage_fast64_3d.hip).
 // Built with -ffp-contract=fast.
 #include "stage_kernels.h"
 
@@ -6,12 +7,14 @@ namespace e4 {
 
 void launch_stage_fast64(const StageArgs& A, dim3 grid, hipStream_t stream, int dims, int flux)
 {
-    launch_stage_mode<ModeFast64>(A, grid, stream, dims, flux);
+    if (dims == 3) launch_stage_fast64_3d(A, grid, stream, flux);
+    else launch_stage_dims<ModeFast64, 2>(A, grid, stream, flux);
 }
 
 void launch_stage_batch_fast64(const BatchArgs& B, int nwg, bool def, hipStream_t stream, int dims, int flux)
 {
-    launch_stage_batch_mode<ModeFast64>(B, nwg, def, stream, dims, flux);
+    if (dims == 3) launch_stage_batch_fast64_3d(B, nwg, def, stream, flux);
+    else launch_stage_batch_dims<ModeFast64, 2>(B, nwg, def, stream, flux);
 }
 
 void launch_extrapolate_ghosts_batch_fast64(const BatchArgs& B, int nwg, hipStream_t stream)

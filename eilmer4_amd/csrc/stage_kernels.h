@@ -631,9 +631,12 @@ __device__ __forceinline__ void stage_tile(int wg)
     constexpr int NHC = 4 * (TX + TY);
     static_assert(NHC <= NT, "one halo cell per thread");
     // 256^3 FP64 1.015 -> 0.994 ms.  (The mixed form gained nothing from it, nor
-    // either form from loading the update's old state before the barrier, and the
-    // exact form has no registers to spare.)
-    constexpr bool AHEAD = std::is_same<M, ModeFast64>::value;
+    // either form from loading the update's old state before the barrier; the
+    // exact form has no registers to spare; nor, with the halo state on top of its
+    // own, has Roe's or AUSM+-up's flux: 128^3 roe, a step: 349 us without, 371 with,
+    // ausm_plus_up 321 and 346.  The near-shock fluxes spill with it, too, but gain:
+    // adaptive_hanel_ausmdv 348 us with, 365 without.)
+    constexpr bool AHEAD = std::is_same<M, ModeFast64>::value && FLUX != FLUX_OTHER;
     unsigned int hpos = HALO_FETCH;
     double hraw[5] = {1.0, 0.0, 0.0, 0.0, 1.0};
     unsigned char hS = 0;
@@ -1291,37 +1294,37 @@ void launch_stage_batch_df(const BatchArgs& B, int nwg, bool def, hipStream_t st
     hipLaunchKernelGGL((stage_kernel<M, TILE_X, TILE_Y, DIMS, FLUX, false, true>), grid, block, 0, stream, B);
 }
 
+template <class M, int DIMS>
+void launch_stage_batch_dims(const BatchArgs& B, int nwg, bool def, hipStream_t stream, int flux)
+{
+    if (flux == FLUX_HLLC) launch_stage_batch_df<M, DIMS, FLUX_HLLC>(B, nwg, def, stream);
+    else if (flux == FLUX_SHOCK) launch_stage_batch_df<M, DIMS, FLUX_SHOCK>(B, nwg, def, stream);
+    else if (flux == FLUX_OTHER) launch_stage_batch_df<M, DIMS, FLUX_OTHER>(B, nwg, def, stream);
+    else launch_stage_batch_df<M, DIMS, FLUX_AUSMDV>(B, nwg, def, stream);
+}
+
 template <class M>
 void launch_stage_batch_mode(const BatchArgs& B, int nwg, bool def, hipStream_t stream, int dims, int flux)
 {
-    if (dims == 3) {
-        if (flux == FLUX_HLLC) launch_stage_batch_df<M, 3, FLUX_HLLC>(B, nwg, def, stream);
-        else if (flux == FLUX_SHOCK) launch_stage_batch_df<M, 3, FLUX_SHOCK>(B, nwg, def, stream);
-        else if (flux == FLUX_OTHER) launch_stage_batch_df<M, 3, FLUX_OTHER>(B, nwg, def, stream);
-        else launch_stage_batch_df<M, 3, FLUX_AUSMDV>(B, nwg, def, stream);
-    } else {
-        if (flux == FLUX_HLLC) launch_stage_batch_df<M, 2, FLUX_HLLC>(B, nwg, def, stream);
-        else if (flux == FLUX_SHOCK) launch_stage_batch_df<M, 2, FLUX_SHOCK>(B, nwg, def, stream);
-        else if (flux == FLUX_OTHER) launch_stage_batch_df<M, 2, FLUX_OTHER>(B, nwg, def, stream);
-        else launch_stage_batch_df<M, 2, FLUX_AUSMDV>(B, nwg, def, stream);
-    }
+    if (dims == 3) launch_stage_batch_dims<M, 3>(B, nwg, def, stream, flux);
+    else launch_stage_batch_dims<M, 2>(B, nwg, def, stream, flux);
 }
 
 // Launch of the stage kernel of mode M for a block of dims dimensions.
+template <class M, int DIMS>
+void launch_stage_dims(const StageArgs& A, dim3 grid, hipStream_t stream, int flux)
+{
+    if (flux == FLUX_HLLC) launch_stage_df<M, DIMS, FLUX_HLLC>(A, grid, stream);
+    else if (flux == FLUX_SHOCK) launch_stage_df<M, DIMS, FLUX_SHOCK>(A, grid, stream);
+    else if (flux == FLUX_OTHER) launch_stage_df<M, DIMS, FLUX_OTHER>(A, grid, stream);
+    else launch_stage_df<M, DIMS, FLUX_AUSMDV>(A, grid, stream);
+}
+
 template <class M>
 void launch_stage_mode(const StageArgs& A, dim3 grid, hipStream_t stream, int dims, int flux)
 {
-    if (dims == 3) {
-        if (flux == FLUX_HLLC) launch_stage_df<M, 3, FLUX_HLLC>(A, grid, stream);
-        else if (flux == FLUX_SHOCK) launch_stage_df<M, 3, FLUX_SHOCK>(A, grid, stream);
-        else if (flux == FLUX_OTHER) launch_stage_df<M, 3, FLUX_OTHER>(A, grid, stream);
-        else launch_stage_df<M, 3, FLUX_AUSMDV>(A, grid, stream);
-    } else {
-        if (flux == FLUX_HLLC) launch_stage_df<M, 2, FLUX_HLLC>(A, grid, stream);
-        else if (flux == FLUX_SHOCK) launch_stage_df<M, 2, FLUX_SHOCK>(A, grid, stream);
-        else if (flux == FLUX_OTHER) launch_stage_df<M, 2, FLUX_OTHER>(A, grid, stream);
-        else launch_stage_df<M, 2, FLUX_AUSMDV>(A, grid, stream);
-    }
+    if (dims == 3) launch_stage_dims<M, 3>(A, grid, stream, flux);
+    else launch_stage_dims<M, 2>(A, grid, stream, flux);
 }
 
 // fluidblock.d:415-431 with PJ_ShockDetector (shockdetectors.d) for every
