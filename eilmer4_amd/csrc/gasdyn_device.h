@@ -68,9 +68,11 @@ __device__ __forceinline__ double rcp_full(double b)
     return fma(r, e, r);
 }
 
-// The square root of a normal positive x far from the ends of the range (the
-// library's also rescales those): Goldschmidt from the hardware's seed, the last
-// step on the exact residual.  Negative x gives a NaN.
+// The square root, without the rescaling by which the library's keeps full accuracy
+// at the ends of the range (below 1e-290 and above 1e290 this one loses bits):
+// Goldschmidt from the hardware's seed, the last step on the exact residual.  Zeros
+// and infinity, whose seeds are not finite, are their own roots; negative x gives a
+// NaN.
 __device__ __forceinline__ double sqrt_mid(double x)
 {
     const double r = __builtin_amdgcn_rsq(x);
@@ -78,7 +80,8 @@ __device__ __forceinline__ double sqrt_mid(double x)
     const double e = fma(-h, g, 0.5);
     g = fma(g, e, g);
     h = fma(h, e, h);
-    return fma(fma(-g, g, x), h, g);
+    const double root = fma(fma(-g, g, x), h, g);
+    return __builtin_amdgcn_class(x, 0x260) ? x : root;   // -0, +0, +inf
 }
 
 // The smaller and larger of two doubles as the instruction gives them (one that
