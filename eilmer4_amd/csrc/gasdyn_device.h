@@ -239,6 +239,12 @@ __device__ __forceinline__ void interp_l2r2_scalar(const L2R2WT<typename M::R>& 
     if (extrema_clipping) {
         qL = clip_limits<M>(qL, qL0, qR0);
         qR = clip_limits<M>(qR, qL0, qR0);
+        if constexpr (M::kFast) {
+            // the comparisons hand on a NaN of the right cell, which min and max
+            // pass over (one of the left cell gives the right cell's value in both)
+            qL = (qR0 != qR0) ? qR0 : qL;
+            qR = (qR0 != qR0) ? qR0 : qR;
+        }
     }
 }
 
