@@ -15,6 +15,7 @@
 
 #include "../../include/e4hip.h"
 #include "aux_kernels.h"
+#include "chunk_rule.h"
 
 namespace {
 
@@ -305,6 +306,12 @@ std::vector<int> tune_key(const BlockH& b)
 
 bool mixed_fluxes() { return g_state.cfg.precision_mode == E4HIP_PRECISION_MIXED; }
 
+double chunk_tail()
+{
+    if (mixed_fluxes()) return 0.0;
+    return (g_state.cfg.precision_mode == E4HIP_PRECISION_FP64_EXACT) ? e4::CHUNK_TAIL_EXACT : e4::CHUNK_TAIL_FP64;
+}
+
 int kchunk_for(const BlockH& b)
 {
     const char* env = getenv("E4HIP_KCHUNK");
@@ -313,8 +320,7 @@ int kchunk_for(const BlockH& b)
     for (const auto& t : g_state.kchunk_tuned)
         if (t.first == key) return t.second;
     long nxy = (long)((b.ni + TILE_X - 1) / TILE_X) * ((b.nj + TILE_Y - 1) / TILE_Y);
-    // aim for >= 2048 workgroups (8 per CU)
-    long chunks = (2048 + nxy - 1) / nxy;
+    const long chunks = e4::untuned_chunks(nxy, b.nk, chunk_tail());
     const int kc = (int)((b.nk + chunks - 1) / chunks);
     return std::min(b.nk, mixed_fluxes() ? std::max(kc, 8) : kc);
 }
@@ -870,10 +876,13 @@ long batch_chunks(const std::vector<const BlockH*>& blks)
     const std::vector<int> key = batch_tune_key(blks);
     for (const auto& t : g_state.kchunk_tuned)
         if (t.first == key) return t.second;
-    long txy = 0;
-    for (const BlockH* b : blks)
-        txy += (long)((b->ni + TILE_X - 1) / TILE_X) * ((b->nj + TILE_Y - 1) / TILE_Y);
-    return (2048 + txy - 1) / txy;
+    long txy = 0, planes = 0;
+    for (const BlockH* b : blks) {
+        const long c = (long)((b->ni + TILE_X - 1) / TILE_X) * ((b->nj + TILE_Y - 1) / TILE_Y);
+        txy += c;
+        planes += c * b->nk;
+    }
+    return e4::untuned_chunks(txy, (planes + txy - 1) / txy, chunk_tail());
 }
 
 int launch_stage_batch(const std::vector<const BlockH*>& blks, const std::vector<unsigned int*>& counters,
