@@ -990,11 +990,11 @@ int launch_stage_batch(const std::vector<const BlockH*>& blks, const std::vector
 
 // Stage sequencing of the thermally perfect path: the same U/dUdt buffer
 // use as launch_stage; the primitive state goes P[0] -> P[1] -> P[0] ...
-// Whether a mixture can use the fast modes' mixture form (tp_gas_device.h).
+// Whether a mixture can use the fast modes' mixture form (tp_gas_device.h): not where
+// its two blend ranges overlap, whose weights that form does not have.
 bool tp_mixture_form(const e4::TPGas& g)
 {
-    return g.shared != 0 && g.curve[0].nseg == e4::TP_FAST_NSEG && g.Tlo <= g.blo[0] && g.bhi[0] < g.blo[1] &&
-           g.bhi[1] <= g.Thi;
+    return g.shared != 0 && g.curve[0].nseg == e4::TP_FAST_NSEG && g.bhi[0] <= g.blo[1];
 }
 
 // The thermally perfect kernels' arguments for one block's stage.

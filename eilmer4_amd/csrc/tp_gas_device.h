@@ -273,7 +273,8 @@ __device__ __forceinline__ TPWeights tp_seg_weights(const TPGas& g, double Tc)
 // Which smooth piece of the fast modes' curve T lies on: below the curve
 // range (0), segment 0 (1), the first blend range (2), segment 1 (3), the
 // second blend range (4), segment 2 (5), above the range (6) -- the same
-// comparisons as tp_seg_weights.  On one piece the energy is one smooth
+// comparisons as tp_seg_weights.  (With a blend range that reaches past an end of
+// the curve's the count differs, but still from piece to piece.)  On one piece the energy is one smooth
 // expression of T (a segment's polynomial and log terms, their linear blend,
 // or the constant-Cp extension).
 __device__ __forceinline__ int tp_curve_piece(const TPGas& g, double T)
