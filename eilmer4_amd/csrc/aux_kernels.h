@@ -102,12 +102,10 @@ __global__ __launch_bounds__(256) void decode_kernel(DecodeArgs A)
     if (nb && __lane_id() == 0) atomicAdd(&A.counters[0], nb);
 }
 
-__global__ void reset_counters_kernel(unsigned int* counters, int n, unsigned long long* smax)
+__global__ void reset_counters_kernel(unsigned int* counters, int n)
 {
     for (int t = threadIdx.x; t < n; t += blockDim.x) counters[t] = 0u;
-    if (threadIdx.x == 0 && smax) *smax = 0ull;
 }
-
 
 // CFL signal from the primitive array (fvcell.d:1624-1661).
 __global__ __launch_bounds__(256) void tp_cfl_kernel(const double* __restrict__ P, long qs, int ni, int nj, int nk,

@@ -25,7 +25,9 @@ inline long untuned_chunks(long cols, long nk, double tail)
     if (tail == 0.0 || (nk + many - 1) / many >= 8) return many;
     auto height = [&](long chunks) { return (nk + chunks - 1) / chunks; };
     auto groups = [&](long chunks) { return cols * ((nk + height(chunks) - 1) / height(chunks)); };
-    auto time = [&](long chunks) { return ((double)height(chunks) + 1.5) * ((double)((groups(chunks) + 767) / 768) + tail); };
+    auto time = [&](long chunks) {
+        return ((double)height(chunks) + 1.5) * ((double)((groups(chunks) + 767) / 768) + tail);
+    };
     return (groups(few) >= 650 && time(few) < time(many)) ? few : many;
 }
 

@@ -1841,7 +1841,7 @@ int e4hip_block_ncells(int blk, long* ncells, int* nq)
 static int run_decode(const BlockH& b, double* fs_dev, unsigned int* nbad)
 {
     hipLaunchKernelGGL(e4::reset_counters_kernel, dim3(1), dim3(64), 0, g_state.stream, g_state.counters,
-                       e4::COUNTER_SLOT, nullptr);
+                       e4::COUNTER_SLOT);
     e4::DecodeArgs D;
     D.U = b.U[0]; D.fs = fs_dev; D.qs = b.qs; D.ncells = b.ncells;
     D.gas = g_state.gases[b.gm].ideal; D.counters = g_state.counters;
@@ -1881,7 +1881,7 @@ int e4hip_block_upload(int blk, const double* U, const double* Tguess)
         HIP_TRY(hipMalloc(&Tg, sizeof(double) * b->ncells));
         HIP_TRY(hipMemcpyAsync(Tg, Tguess, sizeof(double) * b->ncells, hipMemcpyHostToDevice, g_state.stream));
         hipLaunchKernelGGL(e4::reset_counters_kernel, dim3(1), dim3(64), 0, g_state.stream, g_state.counters,
-                       e4::COUNTER_SLOT, nullptr);
+                       e4::COUNTER_SLOT);
         e4::TPArgs A = tp_args_for(*b);
         A.Pout = b->P[0];
         A.guess = g_state.cfg.learned_eos_guess ? g_state.gases[b->gm].guess_dev : nullptr;
@@ -1903,7 +1903,7 @@ int e4hip_block_upload(int blk, const double* U, const double* Tguess)
     unsigned int nbad = 0;
     if (b->general) {
         hipLaunchKernelGGL(e4::reset_counters_kernel, dim3(1), dim3(64), 0, g_state.stream, g_state.counters,
-                           e4::COUNTER_SLOT, nullptr);
+                           e4::COUNTER_SLOT);
         // the decode of an uploaded state is the reference's arithmetic in
         // every precision mode (as decode_kernel's for uniform blocks): the
         // stored flow state must not depend on the mode configured at upload
@@ -2032,7 +2032,7 @@ static int enqueue_step(const int* blks, int nblk, double dt, int ns, unsigned i
     int rc = 0;
     const int nslots = nblk * 3;
     hipLaunchKernelGGL(e4::reset_counters_kernel, dim3(1), dim3(1024), 0, g_state.stream, g_state.step_abort,
-                       ABORT_WORDS + e4::COUNTER_SLOT * nslots, nullptr);
+                       ABORT_WORDS + e4::COUNTER_SLOT * nslots);
     for (int stage = 1; stage <= ns; ++stage) {
         // ghost cells that are stored rather than read through: the x_order-1
         // extrapolation (the other effects are applied on the fly); the ideal

@@ -296,9 +296,9 @@ struct Flux5T {
 // right side mirrored).  AUSMD's momentum is the mass flux times the upwind
 // velocity, and the upwind state is chosen before its enthalpy is formed.  Each
 // denominator has one reciprocal.  About 85 FP64 operations for a face instead
-// of 150, no branch but the rare entropy fix's.  A NaN in any input reaches the
-// mass flux through the positive and negative parts of the velocities, or
-// through the other factors.
+// of 150, no branch but the rare entropy fix's.  A NaN velocity or density reaches the
+// mass flux, a NaN pressure the normal momentum; maxima pass over a NaN sound speed
+// of one side, as the reference's do, and the cell's own decode check counts it.
 __device__ __forceinline__ Flux5T<double> ausmdv_fast64(const FaceStateT<double>& L, const FaceStateT<double>& Rs)
 {
     const double rL = L.rho, pL = L.p, uL = L.vn, aL = L.a, qL = L.RT;

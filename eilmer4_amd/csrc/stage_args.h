@@ -379,8 +379,8 @@ constexpr int TILE_Y = 8;
 constexpr int SD_TX = 62, SD_TY = 8;
 
 // Planes per workgroup of the detector: short enough for about 1024 workgroups
-// (two rounds of what the chip holds; 512 and 2048 measured 3-8 % slower), long enough that the plane read twice at each end
-// of a chunk does not count.
+// (two rounds of what the chip holds; 512 and 2048 measured 3-8 % slower), long
+// enough that the plane read twice at each end of a chunk does not count.
 inline int shock_detect_planes(int ni, int nj, int nk)
 {
     const long cols = (long)((ni + SD_TX - 1) / SD_TX) * ((nj + SD_TY - 1) / SD_TY);

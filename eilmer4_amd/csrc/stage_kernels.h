@@ -515,8 +515,6 @@ template <class M> struct StageOccupancy { static constexpr int waves = E4_STAGE
 template <> struct StageOccupancy<ModeExact> { static constexpr int waves = E4_STAGE_WAVES_EXACT; };
 template <> struct StageOccupancy<ModeMixed> { static constexpr int waves = E4_STAGE_WAVES_MIXED; };
 
-// DEF: the default reconstruction (order 2, limiter, extrema clipping) fixed
-// at compile time; otherwise the three options are read from the arguments.
 // A thread's halo cell of the tile, the same position in every plane: the offset
 // within a plane of the cell it reads -- the cell itself, or the one that a wall,
 // extrapolation or periodic ghost copies -- with flags in the upper bits, or
@@ -548,6 +546,8 @@ __device__ __forceinline__ unsigned int halo_position(KArgs A, int i, int j)
     return h;
 }
 
+// DEF: the default reconstruction (order 2, limiter, extrema clipping) fixed
+// at compile time; otherwise the three options are read from the arguments.
 // One tile of the stage: with BATCH, tile wg of the launch's tile list (the
 // workgroup's own index, or the one it took from the work queue); without,
 // the workgroup's grid position.
@@ -1332,6 +1332,7 @@ void launch_stage_mode(const StageArgs& A, dim3 grid, hipStream_t stream, int di
 // (u_n,right - u_n,left) / min(a_left, a_right) < compression tolerance (the
 // face normal of this axis-aligned grid is a unit axis); a cell is one when
 // any of its faces is.  Ghost neighbours are the ghost-cell effects' states.
+
 // Velocity and sound speed of a cell for the detector: q is the sound speed in
 // ModeExact; in the fast modes its square, which the face test compares with
 // the squared velocity jump (no square root, no division).
@@ -1370,9 +1371,9 @@ __device__ __forceinline__ double sd_min(double aL, double aR) { return (aL < aR
 __device__ __forceinline__ double lane_above(double x)
 {
     const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
-    const unsigned int lo = (unsigned int)__builtin_amdgcn_update_dpp(0, (int)(unsigned int)b, 0x130, 0xf, 0xf, true);
-    const unsigned int hi = (unsigned int)__builtin_amdgcn_update_dpp(0, (int)(unsigned int)(b >> 32), 0x130, 0xf, 0xf, true);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned int)b, 0x130, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned int)(b >> 32), 0x130, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((unsigned long long)(unsigned int)hi << 32) | (unsigned int)lo);
 }
 
 // Where a line's position outside the block (-1, or n) takes its state from, for

@@ -264,10 +264,9 @@ struct TPWeights {
     double b1, b2;
     __device__ __forceinline__ double w(int q) const { return q == 0 ? 1.0 - b1 : (q == 1 ? b1 - b2 : b2); }
 };
-__device__ __forceinline__ double unit_clamp(double x) { return fmin(fmax(x, 0.0), 1.0); }
 __device__ __forceinline__ TPWeights tp_seg_weights(const TPGas& g, double Tc)
 {
-    return TPWeights{unit_clamp((Tc - g.blo[0]) * g.br[0]), unit_clamp((Tc - g.blo[1]) * g.br[1])};
+    return TPWeights{clamp01((Tc - g.blo[0]) * g.br[0]), clamp01((Tc - g.blo[1]) * g.br[1])};
 }
 
 // Which smooth piece of the fast modes' curve T lies on: below the curve
@@ -464,11 +463,12 @@ __device__ __forceinline__ int tp_newton(const TPGas& g, TPState<NSP>& Q, double
 // bisection, or has ended near an end: 3.1 evaluations a solve instead of 5.1
 // on five-species air at 300-8000 K (with the cheaper segment weights, face
 // kernels at 96^3 in FP64 142 -> 112 us, the update 130 -> 120 us; issue-bound).
-// Every lane of the wave goes through the same straight-line body, a finished lane keeping its values: lane-wise exits
-// cost more register copies than the evaluations they saved.  f = e_tgt - u is
-// taken to fall from xMin to xMax, or with `rising` to rise.  Returns 0 with Q.T
-// the root and Q.u the energy of the last iterate, -1 where tp_newton would
-// throw, and 1 where the ends show the order to be the other one.
+// Every lane of the wave goes through the same straight-line body, a finished lane
+// keeping its values: lane-wise exits cost more register copies than the
+// evaluations they saved.  f = e_tgt - u is taken to fall from xMin to xMax, or with
+// `rising` to rise.  Returns 0 with Q.T the root and Q.u the energy of the last
+// iterate, -1 where tp_newton would throw, and 1 where the ends show the order to
+// be the other one.
 template <int NSP>
 __device__ __forceinline__ int tp_newton_fast(const TPGas& g, TPState<NSP>& Q, double Rmix, double e_tgt, double x0,
                                               double xMin, double xMax, bool rising, double tol, int* fevals)
