@@ -32,10 +32,12 @@
 // The FP64 form is bound by FP64 issue: a cell takes about 1100 vector
 // instructions and the kernel keeps the units 70 % busy at the 12 waves a
 // compute unit that 168 registers and 48 KB of LDS allow; a spill or a lower
-// occupancy costs more than the operations it saves.  256^3 ausmdv, one stage:
-// 1.252 ms; 1.065 with the shorter reconstruction and flux; 1.015 with the
-// k direction within the iteration, which ended the spills; 0.994 with the halo
-// cells loaded ahead.
+// occupancy costs more than the operations it saves.  256^3 ausmdv, one stage, as a
+// series on one field at one height: 1.252 ms; 1.065 with the shorter reconstruction
+// and flux; 1.015 with the k direction within the iteration, which ended the spills of
+// ausmdv and hllc (the near-shock fluxes keep 31, Roe's and AUSM+-up's 2); 0.994 with
+// the halo cells loaded ahead.  At its tuned height it takes 0.87 to 0.89 ms.  The
+// mixed form keeps the vector units fully busy (4 waves a SIMD, 100 %).
 #pragma once
 #include "stage_args.h"
 
